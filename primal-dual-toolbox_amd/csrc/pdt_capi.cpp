@@ -2535,7 +2535,7 @@ struct pdt_cnn {
   std::vector<DevBuf> wk, wt;  // packed bf16 weights (forward, backward-data)
   int64_t step = 0;
   int64_t cap = 0;             // pixels the activation buffers hold
-  DevBuf xb, y, dza, dzb, part, lpart;
+  DevBuf y, dza, dzb, part, lpart;
   std::vector<DevBuf> act;     // hidden activations (bf16), nl - 1 of them
   DevBuf ws_x, ws_u, ws_v, ws_ss;  // warm-start input, (u0, v0) and sum of |A^*f|^2
   hipStream_t stream = nullptr;
@@ -2552,61 +2552,71 @@ struct pdt_cnn {
 
   void ensure(int64_t P) {
     if (P <= cap) return;
-    xb.alloc(size_t(P) * ch[0] * 2);
     for (int l = 0; l + 1 < nl; ++l) act[l].alloc(size_t(P) * ch[l + 1] * 2);
-    y.alloc(size_t(P) * ch[nl] * 4);
-    int cmax = 1;
-    for (int c : ch) cmax = std::max(cmax, c);
-    dza.alloc(size_t(P) * cmax * 2);
-    dzb.alloc(size_t(P) * cmax * 2);
-    size_t pf = 0;
-    for (int l = 0; l < nl; ++l) pf = std::max(pf, cnn_wgrad_part_floats(ch[l], ch[l + 1], 1024));
-    part.alloc(pf * 4);
-    lpart.alloc(1024 * sizeof(double));
     cap = P;
   }
 
-  void pack() {
-    for (int l = 0; l < nl; ++l) cnn_pack_weights(stream, W(l), ch[l], ch[l + 1], wk[l].p, l > 0 ? wt[l].p : nullptr);
+  std::vector<CnnLayer> layers() const {
+    std::vector<CnnLayer> ls(nl);
+    for (int l = 0; l < nl; ++l)
+      ls[l] = {W(l), g.as<float>() + off[l], wk[l].p, l > 0 ? wt[l].p : nullptr, nullptr, ch[l], ch[l + 1], 0, 0, 0};
+    return ls;
   }
 
-  // y = net(x) for P = n h w pixels (x: fp32 NHWC on the device)
-  void forward(const float* x, int n, int h, int wd) {
-    const int64_t P = int64_t(n) * h * wd;
-    ensure(P);
-    cnn_to_bf16(stream, x, xb.p, P * ch[0]);
-    const void* in = xb.p;
-    for (int l = 0; l < nl; ++l) {
-      const bool last = l + 1 == nl;
-      void* out = last ? y.p : act[l].p;
-      cnn_conv_forward(stream, ch[l], ch[l + 1], !last, in, wk[l].p, b(l), out, n, h, wd);
-      in = out;
-    }
+  void pack() { cnn_pack_weights(stream, layers().data(), nl); }
+
+  // hidden activations of P = n h w pixels (x: fp32 NHWC on the device)
+  const void* hidden(const float* x, int n, int h, int wd) {
+    ensure(int64_t(n) * h * wd);
+    cnn_conv_first(stream, x, wk[0].p, b(0), act[0].p, n, h, wd);
+    for (int l = 1; l + 1 < nl; ++l) cnn_conv_hidden(stream, act[l - 1].p, wk[l].p, b(l), act[l].p, n, h, wd);
+    return act[nl - 2].p;
+  }
+
+  // out = net(x)
+  void forward(const float* x, float* out, int n, int h, int wd) {
+    const void* in = hidden(x, n, h, wd);
+    cnn_conv_last(stream, in, wk[nl - 1].p, b(nl - 1), out, n, h, wd);
     HIPC(hipGetLastError());
   }
 
-  // loss and gradient (into g) of the last forward against t
-  double backward(const float* t, int n, int h, int wd) {
+  // loss of net(x) against t and its gradient (into g)
+  double loss_grad(const float* x, const float* t, int n, int h, int wd) {
     const int64_t P = int64_t(n) * h * wd, M = P * ch[nl];
-    const int nb = cnn_mse_blocks(M);
+    const void* last = hidden(x, n, h, wd);
+    int cmax = 8;  // the output gradient is padded to 8 channels
+    for (int l = 1; l < nl; ++l) cmax = std::max(cmax, ch[l]);
+    dza.ensure(size_t(P) * cmax * 2);
+    dzb.ensure(size_t(P) * cmax * 2);
+    std::vector<CnnLayer> ls = layers();
+    size_t pf = 0;
+    for (int l = 0; l < nl; ++l) pf += cnn_wgrad_part_floats(ch[l], ch[l + 1], n, h, wd);
+    part.ensure(pf * 4);
+    float* pp = part.as<float>();
+    for (int l = 0; l < nl; ++l) {
+      ls[l].part = pp;
+      pp += cnn_wgrad_part_floats(ch[l], ch[l + 1], n, h, wd);
+    }
+    const int nb = cnn_mse_blocks(n, h, wd);
+    lpart.ensure(size_t(nb) * sizeof(double));
     void* dz = dza.p;
     void* dzn = dzb.p;
-    cnn_mse(stream, y.as<float>(), t, M, dz, lpart.as<double>(), nb);
-    const int nblk = cnn_wgrad_blocks(n, h, wd);
+    cnn_conv_last_mse(stream, last, wk[nl - 1].p, b(nl - 1), t, dz, lpart.as<double>(), n, h, wd);
     for (int l = nl - 1; l >= 0; --l) {
-      const void* in = l == 0 ? xb.p : act[l - 1].p;
-      cnn_conv_wgrad(stream, ch[l], ch[l + 1], in, dz, part.as<float>(), nblk, g.as<float>() + off[l], n, h, wd);
+      const void* in = l == 0 ? static_cast<const void*>(x) : act[l - 1].p;
+      cnn_conv_wgrad(stream, ls[l], in, dz, n, h, wd);
       if (l > 0) {
-        cnn_conv_backward_data(stream, ch[l], ch[l + 1], dz, wt[l].p, act[l - 1].p, dzn, n, h, wd);
+        cnn_conv_backward_data(stream, ch[l + 1], dz, wt[l].p, act[l - 1].p, dzn, n, h, wd);
         std::swap(dz, dzn);
       }
     }
+    cnn_reduce_grads(stream, ls.data(), nl);
     HIPC(hipGetLastError());
     std::vector<double> lp(nb);
     HIPC(hipMemcpyAsync(lp.data(), lpart.p, nb * sizeof(double), hipMemcpyDeviceToHost, stream));
     HIPC(hipStreamSynchronize(stream));
     double ss = 0;
-    for (double x : lp) ss += x;
+    for (double v : lp) ss += v;
     return ss / (2.0 * double(M));
   }
 
@@ -2663,7 +2673,7 @@ int pdt_cnn_create(int cin, int width, int depth, int cout, pdt_cnn** out) {
     net->act.resize(depth - 1);
     for (int l = 0; l < depth; ++l) {
       net->wk[l].alloc(cnn_wk_elems(net->ch[l], net->ch[l + 1]) * 2);
-      if (l > 0) net->wt[l].alloc(cnn_wt_elems(net->ch[l], net->ch[l + 1]) * 2);
+      if (l > 0) net->wt[l].alloc(cnn_wk_elems(net->ch[l + 1], net->ch[l]) * 2);
     }
     run_zero(net->stream, net->w.p, net->np * 4);
     run_zero(net->stream, net->m.p, net->np * 4);
@@ -2714,8 +2724,7 @@ int pdt_cnn_forward(pdt_cnn* net, const pdt_array* x, pdt_array* y, int n, int h
     const int64_t P = int64_t(n) * h * w;
     const float* xp = cnn_tensor(x, P * net->ch[0], "x");
     float* yp = const_cast<float*>(cnn_tensor(y, P * net->ch[net->nl], "y"));
-    net->forward(xp, n, h, w);
-    HIPC(hipMemcpyAsync(yp, net->y.p, size_t(P) * net->ch[net->nl] * 4, hipMemcpyDeviceToDevice, net->stream));
+    net->forward(xp, yp, n, h, w);
     HIPC(hipStreamSynchronize(net->stream));
   });
 }
@@ -2729,8 +2738,7 @@ int pdt_cnn_loss_grad(pdt_cnn* net, const pdt_array* x, const pdt_array* t, int 
     const float* xp = cnn_tensor(x, P * net->ch[0], "x");
     const float* tp = cnn_tensor(t, P * net->ch[net->nl], "t");
     if (grad_host && n_grad != net->np) fail(PDT_ERR_SIZE, "gradient buffer must hold every parameter");
-    net->forward(xp, n, h, w);
-    const double l = net->backward(tp, n, h, w);
+    const double l = net->loss_grad(xp, tp, n, h, w);
     if (loss) *loss = l;
     if (grad_host) HIPC(hipMemcpy(grad_host, net->g.p, net->np * 4, hipMemcpyDeviceToHost));
   });
@@ -2752,8 +2760,7 @@ int pdt_cnn_train_step(pdt_cnn* net, const pdt_array* x, const pdt_array* t, int
     const int64_t P = int64_t(n) * h * w;
     const float* xp = cnn_tensor(x, P * net->ch[0], "x");
     const float* tp = cnn_tensor(t, P * net->ch[net->nl], "t");
-    net->forward(xp, n, h, w);
-    const double l = net->backward(tp, n, h, w);
+    const double l = net->loss_grad(xp, tp, n, h, w);
     if (loss) *loss = l;
     net->adam(*opt);
     HIPC(hipStreamSynchronize(net->stream));
@@ -2784,7 +2791,8 @@ int pdt_solver_warm_start(pdt_solver* s, pdt_cnn* net) {
     cnn_ws_pack(s->stream, s->atf.p, n, net->ws_ss.as<double>(), net->ws_x.as<float>());
     HIPC(hipEventRecord(net->ev_in, s->stream));
     HIPC(hipStreamWaitEvent(net->stream, net->ev_in, 0));
-    net->forward(net->ws_x.as<float>(), 1, H, W);
+    net->y.ensure(size_t(n) * 6 * 4);
+    net->forward(net->ws_x.as<float>(), net->y.as<float>(), 1, H, W);
     cnn_ws_unpack(net->stream, net->ws_x.as<float>(), net->y.as<float>(), n, net->ws_ss.as<double>(), net->ws_u.p,
                   net->ws_v.p);
     HIPC(hipGetLastError());

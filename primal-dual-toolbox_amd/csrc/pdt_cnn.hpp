@@ -11,26 +11,48 @@ namespace pdt {
 
 // Layer shapes with kernels: 2 -> 32, 32 -> 32, 32 -> 6.
 bool cnn_layer_supported(int cin, int cout);
-// Packed bf16 weight sizes (elements) of a layer, forward and backward-data.
+// A layer as the kernels that take the whole network in one launch see it.
+struct CnnLayer {
+  const float* w;  // fp32 master W[tap][co][ci], b
+  float* g;        // its gradient, same layout
+  void* wk;        // packed bf16 weights
+  void* wt;        // packed bf16 weights of the backward-data pass (null: first layer)
+  float* part;     // per-block partial gradients (cnn_wgrad_part_floats)
+  int cin, cout;
+  int nblk;        // partials written by cnn_conv_wgrad
+  int nk, nt;      // elements of wk, wt (set by cnn_pack_weights)
+};
+constexpr int kCnnLayers = 8;  // layers per launch
+struct CnnLayers {
+  CnnLayer l[kCnnLayers];
+};
+
+// Elements of the packed bf16 weights of a convolution cin -> cout (the
+// backward-data pass of a layer is one of its output to its input channels).
 size_t cnn_wk_elems(int cin, int cout);
-size_t cnn_wt_elems(int cin, int cout);
-// fp32 master W[tap][co][ci] -> packed bf16 copies (wt may be null).
-void cnn_pack_weights(hipStream_t st, const float* W, int cin, int cout, void* wk, void* wt);
-void cnn_to_bf16(hipStream_t st, const float* x, void* y, int64_t n);
-// out = conv(in) + b, then ReLU and bf16 (relu) or fp32 (last layer).
-void cnn_conv_forward(hipStream_t st, int cin, int cout, bool relu, const void* in, const void* wk, const float* b,
-                      void* out, int n, int h, int w);
-// din = (conv^T dz) * [act > 0], bf16.
-void cnn_conv_backward_data(hipStream_t st, int cin, int cout, const void* dz, const void* wt, const void* act,
-                            void* din, int n, int h, int w);
-// grad (master layout W then b) of one layer; part holds cnn_wgrad_part_floats.
-int cnn_wgrad_blocks(int n, int h, int w);
-size_t cnn_wgrad_part_floats(int cin, int cout, int nblk);
-void cnn_conv_wgrad(hipStream_t st, int cin, int cout, const void* in, const void* dz, float* part, int nblk,
-                    float* grad, int n, int h, int w);
-// MSE 1/(2m) sum (y - t)^2: fp64 per-block partials and dz = (y - t) / m (bf16).
-int cnn_mse_blocks(int64_t m);
-void cnn_mse(hipStream_t st, const float* y, const float* t, int64_t m, void* dz, double* part, int nblk);
+// fp32 master weights -> packed bf16 copies.
+void cnn_pack_weights(hipStream_t st, const CnnLayer* ls, int count);
+// The layers of the forward pass: relu(conv(x) + b) in bf16 from the fp32
+// input (2 -> 32), between hidden activations (32 -> 32), and the fp32
+// output conv(in) + b (32 -> 6).
+void cnn_conv_first(hipStream_t st, const float* x, const void* wk, const float* b, void* out, int n, int h, int w);
+void cnn_conv_hidden(hipStream_t st, const void* in, const void* wk, const float* b, void* out, int n, int h, int w);
+void cnn_conv_last(hipStream_t st, const void* in, const void* wk, const float* b, float* y, int n, int h, int w);
+// The last layer of a training pass: y = conv(in) + b is not stored but
+// compared with t: the loss 1/(2m) sum (y - t)^2 over the m = 6 n h w outputs
+// as cnn_mse_blocks fp64 partial sums, and dz = (y - t) / m in bf16, padded to
+// 8 channels.
+void cnn_conv_last_mse(hipStream_t st, const void* in, const void* wk, const float* b, const float* t, void* dz,
+                       double* part, int n, int h, int w);
+int cnn_mse_blocks(int n, int h, int w);
+// din = (conv^T dz) * [act > 0], bf16, of a layer 32 -> cout.
+void cnn_conv_backward_data(hipStream_t st, int cout, const void* dz, const void* wt, const void* act, void* din, int n,
+                            int h, int w);
+// Per-block partial gradients of a layer (in: bf16, fp32 for the first), and
+// their sums in every layer's g.
+size_t cnn_wgrad_part_floats(int cin, int cout, int n, int h, int w);
+void cnn_conv_wgrad(hipStream_t st, CnnLayer& L, const void* in, const void* dz, int n, int h, int w);
+void cnn_reduce_grads(hipStream_t st, const CnnLayer* ls, int count);
 // One Adam update; c1 = 1 - b1^t, c2 = 1 - b2^t.
 void cnn_adam(hipStream_t st, float* w, const float* g, float* m, float* v, int64_t n, float lr, float b1, float b2,
               float eps, float c1, float c2);

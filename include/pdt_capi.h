@@ -226,7 +226,9 @@ typedef struct pdt_tiles {
   int32_t wpc[4];  /* workgroups per CU, 0 = no cap: forward row, column,
                       adjoint row and denoising passes                          */
   int32_t tb_x, tb_y, tb_k; /* ROF or TGV denoising, one slice: tb_k
-                      iterations per launch on tb_x x tb_y tiles held in LDS
+                      iterations per launch on tiles of tb_x x tb_y pixels
+                      and a halo of tb_k, cut to the 64 columns and the rows
+                      (32 or 64) a workgroup holds
                       (tb_k 0: one iteration per pair of launches)               */
   int32_t dual_px; /* TGV denoising: pixels per thread of the dual step, 1 or 2
                       (2 needs even widths; 0: the default, 2 where possible)   */
@@ -256,7 +258,7 @@ PDT_API int pdt_autotune(pdt_solver** solvers, int count, int reps, pdt_tiles* o
  * where a single slice's straight-line adjoint path fits, else cb), values
  * above a shape's limit are clamped; wpc in
  * [0, 6]; tb_k <= 0 turns the blocked denoising launches off, and tiles
- * that do not fit the LDS are not used.  The next solve of the same shape
+ * whose halo leaves no interior are not used.  The next solve of the same shape
  * uses it. */
 PDT_API int pdt_set_tiles(pdt_solver** solvers, int count, const pdt_tiles* tiles);
 

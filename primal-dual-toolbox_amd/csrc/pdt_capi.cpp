@@ -212,11 +212,8 @@ int max_cg(int dt, int Hk, int nc) {
   return cg;
 }
 // Default tiles before any autotuning: 4 coils per row item, 2 columns per
-// column group; temporally blocked ROF launches of 8 iterations on 32 x 16
-// tiles.
+// column group (temporally blocked denoising: block_choose).
 constexpr int kDefaultCb = 4, kDefaultCg = 2;
-constexpr int kDefaultTvBlock[3] = {32, 16, 8};
-constexpr int kDefaultTgvBlock[3] = {16, 16, 4};
 
 }  // namespace
 
@@ -917,13 +914,12 @@ struct Engine {
       // double: 12.2 against 9.5 us per dual step)
       const int dpx = force_dpx > 0 ? force_dpx : tv.dual_px > 0 ? tv.dual_px : is_dbl(dtype) ? 1 : 2;
       pair_duals = dpx == 2;
-      // temporally blocked launches: one slice only, tiles that fit the LDS
-      const int* tb = force_tb[2] >= 0 ? force_tb
-                      : tv.tb[2] >= 0  ? tv.tb
-                      : kind == PDT_SOLVER_TGV ? kDefaultTgvBlock
-                                               : kDefaultTvBlock;
+      // temporally blocked launches: one slice only
+      int chosen[3];
+      block_choose(kind, dt, fp16, sv[0]->W, sv[0]->H, chosen);
+      const int* tb = force_tb[2] >= 0 ? force_tb : tv.tb[2] >= 0 ? tv.tb : chosen;
       if ((kind == PDT_SOLVER_TV || kind == PDT_SOLVER_TGV) && ns == 1 &&
-          block_fits(kind, dt, tb[0], tb[1], tb[2], init_kernel_attrs())) {
+          block_shape(kind, dt, sv[0]->W, sv[0]->H, tb[0], tb[1], tb[2]).grid > 0) {
         L.tb_x = tb[0];
         L.tb_y = tb[1];
         L.tb_k = tb[2];
@@ -1219,8 +1215,6 @@ struct Engine {
         x.pair = x.adj_fused && ndual > 0 && dt == DT_C64 && !unpaired;
       }
       if (!(dense && (kind == PDT_SOLVER_TV || kind == PDT_SOLVER_TGV))) x.tb_x = x.tb_y = x.tb_k = 0;
-      x.tb_w = hs[groups[r.g][0]].W;
-      x.tb_h = hs[groups[r.g][0]].H;
       listed_items += r.nrow + r.nrg + r.nrga + r.ncol;
       G.push_back(x);
     }
@@ -1340,19 +1334,24 @@ struct Engine {
   // first: the iterations start a solve (paired iterations take the T1 of
   // the first one from the forward row pass, later chunks from the last
   // adjoint row pass of the chunk before).
-  // With temporally blocked ROF launches, the iterations before the gap
-  // iteration run as pairs of launches of tb_k iterations each (the state
-  // goes to the second copy and back), the rest one iteration at a time.
+  // With temporally blocked launches, the iterations before the gap
+  // iteration run as pairs of launches of at most tb_k iterations each.
   void enqueue(int len, bool gap, bool first = true) {
     const int dt = dtk();
     if (blocked()) {
       const int k = G[0].tb_k;
-      int plain = len - (gap ? 1 : 0);
-      for (; plain >= 2 * k; plain -= 2 * k) {
-        run_block(G[0], kind, dt, fp16, 0);
-        run_block(G[0], kind, dt, fp16, 1);
+      // pairs of launches (the state goes to its second copy and back): as
+      // few as hold the iterations with at most k each, of equal lengths
+      int plain = len - (gap ? 1 : 0), launches = 2 * ((plain + 2 * k - 1) / (2 * k));
+      if (launches > plain) {  // one iteration, or an odd number one at a time
+        iteration(false);
+        launches = --plain;
       }
-      for (int i = 0; i < plain; ++i) iteration(false);
+      for (int i = 0, done = 0; i < launches; ++i) {
+        const int n = (plain - done) / (launches - i);
+        run_block(G[0], hs[0], kind, dt, fp16, i & 1, n);
+        done += n;
+      }
       if (gap) {
         iteration(true);
         run_gap_reduce(L, kind, dt);
@@ -1426,12 +1425,10 @@ struct Engine {
     // not hidden); the gap is evaluated at the multiples of gap_every.
     constexpr unsigned kChunk = 50;
     unsigned chunk = std::min<unsigned>(gap ? gap_every : total, kChunk);
-    // blocked ROF launches come in pairs of tb_k iterations: chunks of a
-    // multiple of 2 tb_k leave no iterations to the one-iteration kernels
-    if (blocked()) {
-      const unsigned pair = 2u * unsigned(G[0].tb_k);
-      chunk = std::max(pair, chunk - chunk % pair);
-    }
+    // blocked launches hold tb_k iterations each: chunks of kBlockLaunches
+    // launches (the start of the next graph costs about one of them)
+    constexpr unsigned kBlockLaunches = 24;
+    if (blocked()) chunk = std::min<unsigned>(gap ? gap_every : total, kBlockLaunches * unsigned(G[0].tb_k));
     const bool use_graph = sv[0]->prm.use_graph != 0;
     std::vector<double> stop_ms(ns, -1.0);  // batched solves: time from the start to each slice's stop
     reset_ctl();
@@ -2117,8 +2114,8 @@ void profile_engine(std::vector<pdt_solver*> sv, int reps, pdt_kernel_prof* out,
         SetupLock lk(g_setup_mu);
         HIPC(hipStreamBeginCapture(e.stream, hipStreamCaptureModeThreadLocal));
         for (int r = 0; r < reps; ++r) {
-          run_block(e.G[0], e.kind, e.dtk(), e.fp16, 0);
-          run_block(e.G[0], e.kind, e.dtk(), e.fp16, 1);
+          run_block(e.G[0], e.hs[0], e.kind, e.dtk(), e.fp16, 0, e.G[0].tb_k);
+          run_block(e.G[0], e.hs[0], e.kind, e.dtk(), e.fp16, 1, e.G[0].tb_k);
         }
         HIPC(hipStreamEndCapture(e.stream, &graph));
         HIPC(hipGraphInstantiate(&ge, graph, nullptr, nullptr, 0));
@@ -2264,12 +2261,12 @@ double time_iteration(Engine& e, int reps) {
     hipEvent_t e0, e1;
     HIPC(hipEventCreate(&e0));
     HIPC(hipEventCreate(&e1));
-    run_block(e.G[0], e.kind, e.dtk(), e.fp16, 0);
-    run_block(e.G[0], e.kind, e.dtk(), e.fp16, 1);
+    run_block(e.G[0], e.hs[0], e.kind, e.dtk(), e.fp16, 0, e.G[0].tb_k);
+    run_block(e.G[0], e.hs[0], e.kind, e.dtk(), e.fp16, 1, e.G[0].tb_k);
     HIPC(hipEventRecord(e0, e.stream));
     for (int r = 0; r < reps; ++r) {
-      run_block(e.G[0], e.kind, e.dtk(), e.fp16, 0);
-      run_block(e.G[0], e.kind, e.dtk(), e.fp16, 1);
+      run_block(e.G[0], e.hs[0], e.kind, e.dtk(), e.fp16, 0, e.G[0].tb_k);
+      run_block(e.G[0], e.hs[0], e.kind, e.dtk(), e.fp16, 1, e.G[0].tb_k);
     }
     HIPC(hipEventRecord(e1, e.stream));
     HIPC(hipEventSynchronize(e1));
@@ -2326,17 +2323,11 @@ int pdt_autotune(pdt_solver** solvers, int count, int reps, pdt_tiles* out, doub
       for (int rpi : {1, 2, 4, 8})
         for (int dpx : sv[0]->kind == PDT_SOLVER_TGV ? std::vector<int>{1, 2} : std::vector<int>{0})
           cand.push_back({{0, 0, rpi, 0}, {0, 0, 0}, dpx});
-      if (sv[0]->kind == PDT_SOLVER_TV && sv.size() == 1)
-        for (const auto& tb : std::vector<std::array<int, 3>>{
-                 {16, 16, 4}, {16, 16, 6}, {32, 16, 4}, {32, 16, 8}, {32, 32, 8}, {64, 32, 8}, {32, 32, 12},
-                 {64, 64, 8}, {64, 64, 16}})
-          cand.push_back({{0, 0, 1, 0}, tb, 0});
-      // TGV holds 8 planes per tile pixel in LDS: smaller tiles and halos
-      if (sv[0]->kind == PDT_SOLVER_TGV && sv.size() == 1)
-        for (const auto& tb : std::vector<std::array<int, 3>>{
-                 {16, 8, 2}, {16, 16, 2}, {16, 16, 4}, {32, 8, 2}, {32, 16, 2}, {32, 16, 4}, {32, 32, 2}, {32, 32, 4},
-                 {32, 32, 6}, {48, 32, 4}, {64, 16, 4}, {64, 32, 3}})
-          cand.push_back({{0, 0, 1, 0}, tb, 0});
+      // one slice: the blocked tiles of whole waves of rows
+      if (sv.size() == 1)
+        for (int k : kBlockIterations)
+          for (int waves : kBlockWaves)
+            if (waves * kBlockRows > 2 * k) cand.push_back({{0, 0, 1, 0}, {64 - 2 * k, waves * kBlockRows - 2 * k, k}, 0});
     }
     auto engine = [&](const Cand& c, const int (&wpc)[4]) {
       auto e = std::make_unique<Engine>();

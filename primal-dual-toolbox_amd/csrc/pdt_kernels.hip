@@ -33,126 +33,9 @@
 
 #include "pdt_desc.hpp"
 #include "pdt_launch.hpp"
+#include "pdt_pixel.hpp"
 
 namespace pdt {
-
-// ---------------------------------------------------------------------------
-// Pixel arithmetic
-// ---------------------------------------------------------------------------
-template <class R>
-struct alignas(2 * sizeof(R)) Cx {
-  R re, im;
-};
-
-template <class R> __device__ __forceinline__ Cx<R> operator+(Cx<R> a, Cx<R> b) { return {a.re + b.re, a.im + b.im}; }
-template <class R> __device__ __forceinline__ Cx<R> operator-(Cx<R> a, Cx<R> b) { return {a.re - b.re, a.im - b.im}; }
-template <class R> __device__ __forceinline__ Cx<R> operator-(Cx<R> a) { return {-a.re, -a.im}; }
-// Complex products with explicit fused multiply-adds: left to the compiler,
-// the contraction of a.re b.im + a.im b.re fused one product in one kernel
-// and the other in another (both are one rounding short of two), so the same
-// product of the same values differed in the last bit between kernels.
-template <class R> __device__ __forceinline__ Cx<R> operator*(Cx<R> a, Cx<R> b) {
-  return {fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re)};
-}
-template <class R> __device__ __forceinline__ Cx<R> operator*(R s, Cx<R> a) { return {s * a.re, s * a.im}; }
-template <class R> __device__ __forceinline__ Cx<R> operator*(Cx<R> a, R s) { return {s * a.re, s * a.im}; }
-template <class R> __device__ __forceinline__ Cx<R> operator/(Cx<R> a, R s) { return {a.re / s, a.im / s}; }
-// a * x + y with one rounding per component.  The denoising primal steps
-// write div + lambda f with it, so that every kernel rounds it the same way
-// (left to the compiler, a kernel that holds f across iterations computed
-// lambda f once, rounded, and the one-iteration kernels fused it).
-template <class R> __device__ __forceinline__ R fmadd(R a, R x, R y) { return fma(a, x, y); }
-template <class R> __device__ __forceinline__ Cx<R> fmadd(R a, Cx<R> x, Cx<R> y) {
-  return {fma(a, x.re, y.re), fma(a, x.im, y.im)};
-}
-// c ? a : b, component-wise (a select, not a branch)
-template <class R> __device__ __forceinline__ Cx<R> csel(bool c, Cx<R> a, Cx<R> b) {
-  return {c ? a.re : b.re, c ? a.im : b.im};
-}
-// a * conj(b)
-template <class R> __device__ __forceinline__ Cx<R> mulconj(Cx<R> a, Cx<R> b) {
-  return {fma(a.re, b.re, a.im * b.im), fma(a.im, b.re, -(a.re * b.im))};
-}
-
-template <class P> struct PT { using R = P; static constexpr bool cplx = false; };
-template <class R> struct PT<Cx<R>> { using Rt = R; using R_ = R; static constexpr bool cplx = true; };
-template <class P> struct RealOf { using T = P; };
-template <class R> struct RealOf<Cx<R>> { using T = R; };
-
-template <class P> __device__ __forceinline__ P pzero() { return P(0); }
-template <> __device__ __forceinline__ Cx<float> pzero<Cx<float>>() { return {0.f, 0.f}; }
-template <> __device__ __forceinline__ Cx<double> pzero<Cx<double>>() { return {0.0, 0.0}; }
-
-__device__ __forceinline__ float abs2(float a) { return a * a; }
-__device__ __forceinline__ double abs2(double a) { return a * a; }
-template <class R> __device__ __forceinline__ R abs2(Cx<R> a) { return fma(a.re, a.re, a.im * a.im); }  // (as the products above)
-__device__ __forceinline__ double dabs2(float a) { return double(a) * double(a); }
-__device__ __forceinline__ double dabs2(double a) { return a * a; }
-template <class R> __device__ __forceinline__ double dabs2(Cx<R> a) {
-  return double(a.re) * double(a.re) + double(a.im) * double(a.im);
-}
-__device__ __forceinline__ double redot(float a, float b) { return double(a) * double(b); }
-__device__ __forceinline__ double redot(double a, double b) { return a * b; }
-template <class R> __device__ __forceinline__ double redot(Cx<R> a, Cx<R> b) {
-  return double(a.re) * double(b.re) + double(a.im) * double(b.im);
-}
-
-// fp16 storage of the TGV duals (compute stays in the pixel type).
-template <class P> struct Half;
-template <> struct Half<float> { using T = _Float16; };
-template <> struct Half<Cx<float>> { using T = Cx<_Float16>; };
-template <> struct Half<double> { using T = double; };
-template <> struct Half<Cx<double>> { using T = Cx<double>; };
-
-// Device memory reached through the slice descriptors is addressed with
-// global-address-space pointers (gptr): loads and stores through them compile
-// to global_* instructions with a scalar base, where generic pointers give
-// flat_* ones, which also count against the LDS wait counter (so every LDS
-// wait of an FFT stage would wait for the outstanding register prefetches).
-// (The host pass of the same source, which only checks device code, keeps
-// generic pointers.)
-#if defined(__HIP_DEVICE_COMPILE__)
-template <class T> using G = __attribute__((address_space(1))) T;
-template <class T> struct NoAS { using type = T; };
-template <class T> struct NoAS<G<T>> { using type = T; };
-#else
-template <class T> using G = T;
-template <class T> struct NoAS { using type = T; };
-#endif
-template <class T> using Plain = std::remove_const_t<typename NoAS<T>::type>;
-template <class T>
-__device__ __forceinline__ G<T>* gptr(const void* p) {
-  return (G<T>*)(const_cast<void*>(p));
-}
-
-// Element access of a plane stored as S (get/put take any pointer to S).
-template <class P, class S> struct Ld {
-  template <class A> static __device__ __forceinline__ P get(A* a, size_t i) { return a[i]; }
-  template <class A> static __device__ __forceinline__ void put(A* a, size_t i, P v) { a[i] = v; }
-};
-// The value stored is the float result rounded to nearest half: the empty
-// register constraint keeps the compiler from fusing the product that
-// produced it with the conversion (a mixed-precision FMA rounds once, straight
-// to half), so every kernel stores the same halves.
-__device__ __forceinline__ _Float16 to_half(float v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm("" : "+v"(v));
-#endif
-  return _Float16(v);
-}
-template <> struct Ld<float, _Float16> {
-  template <class A> static __device__ __forceinline__ float get(A* a, size_t i) { return float(a[i]); }
-  template <class A> static __device__ __forceinline__ void put(A* a, size_t i, float v) { a[i] = to_half(v); }
-};
-template <> struct Ld<Cx<float>, Cx<_Float16>> {
-  template <class A> static __device__ __forceinline__ Cx<float> get(A* a, size_t i) {
-    Cx<_Float16> h = a[i];
-    return {float(h.re), float(h.im)};
-  }
-  template <class A> static __device__ __forceinline__ void put(A* a, size_t i, Cx<float> v) {
-    a[i] = Cx<_Float16>{to_half(v.re), to_half(v.im)};
-  }
-};
 
 // ---------------------------------------------------------------------------
 // Block reductions (wave64 shuffles, then the 4 waves in a fixed order)
@@ -769,11 +652,6 @@ __device__ __forceinline__ P dmy(const S* a, int y, size_t i, int W, int H) {
   return y > 0 ? d : c;
 }
 
-// 1 / x: the hardware reciprocal (within 1 ulp) in single precision, a
-// correctly rounded division in double precision.
-template <class R> __device__ __forceinline__ R rcp(R x) { return R(1) / x; }
-template <> __device__ __forceinline__ float rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
-
 template <class R>
 __device__ __forceinline__ R sched_alpha(const SliceDev& d, double a_start, double a_end, int k) {
   if (!d.schedule) return R(a_start);
@@ -782,55 +660,11 @@ __device__ __forceinline__ R sched_alpha(const SliceDev& d, double a_start, doub
   return exp(dk / dmax * log(R(a_end)) + (dmax - dk) / dmax * log(R(a_start)));
 }
 
-// The arithmetic of the dual step at one pixel, on values: c = ubar, uxp /
-// uyp = ubar at the forward neighbours (c itself at the last column / row);
-// TGV: vx0, vy0 = vbar, vxx = vbar_x and vyx = vbar_y at the x neighbour,
-// vxy, vyy at the y neighbour.  Updates p (and q) in place, with optional
-// gap terms t[0] += |grad ub - vb|, t[1] += |E vb|_F, t[2] += Re<grad ub -
-// vb, p> + Re<E vb, q>_F (TGV_dual_p_kernel / TGV_dual_q_kernel /
-// TV_dual_p_kernel).  ia0, ia1 = 1 / alpha0, 1 / alpha1 (TGV only).
-template <class P, bool TGV, bool GAP>
-__device__ __forceinline__ void dual_math(P c, P uxp, P uyp, P vx0, P vy0, P vxx, P vyx, P vxy, P vyy, P& px, P& py,
-                                          P& qxx, P& qyy, P& qxy, typename RealOf<P>::T sigma,
-                                          typename RealOf<P>::T ia0, typename RealOf<P>::T ia1, double* t) {
-  using R = typename RealOf<P>::T;
-  P tx = uxp - c, ty = uyp - c;
-  if (TGV) {
-    tx = tx - vx0;
-    ty = ty - vy0;
-    const P exx = vxx - vx0;
-    const P eyy = vyy - vy0;
-    const P exy = R(0.5) * (vxy - vx0 + vyx - vy0);
-    const P bxx = qxx + sigma * exx;
-    const P byy = qyy + sigma * eyy;
-    const P bxy = qxy + sigma * exy;
-    const R qn = sqrt(abs2(bxx) + abs2(byy) + R(2) * abs2(bxy));
-    const R sq = rcp(fmax(R(1), qn * ia0));
-    qxx = bxx * sq;
-    qyy = byy * sq;
-    qxy = bxy * sq;
-    if (GAP) {
-      t[1] += sqrt(dabs2(exx) + dabs2(eyy) + 2.0 * dabs2(exy));
-      t[2] += redot(exx, qxx) + redot(eyy, qyy) + 2.0 * redot(exy, qxy);
-    }
-  }
-  const P ax = px + sigma * tx;
-  const P ay = py + sigma * ty;
-  const R pn = sqrt(abs2(ax) + abs2(ay));
-  const R sp = rcp(fmax(R(1), TGV ? pn * ia1 : pn));
-  px = ax * sp;
-  py = ay * sp;
-  if (GAP) {
-    t[0] += sqrt(dabs2(tx) + dabs2(ty));
-    t[2] += redot(tx, px) + redot(ty, py);
-  }
-}
-
 // Dual ascent + projection of p (and q) at one pixel (dual_math on the
 // pixel's values in memory).
 template <class P, class S, bool TGV, bool GAP>
 __device__ __forceinline__ void dual_pixel(const SliceDev& d, int x, int y, typename RealOf<P>::T sigma,
-                                           typename RealOf<P>::T ia0, typename RealOf<P>::T ia1,
+                                           typename RealOf<P>::T w0, typename RealOf<P>::T w1,
                                            double* t) {
   using L = Ld<P, S>;
   const int W = d.W, H = d.H;
@@ -859,8 +693,8 @@ __device__ __forceinline__ void dual_pixel(const SliceDev& d, int x, int y, type
     qxy = L::get(qxyp, i);
   }
   P pxv = L::get(px, i), pyv = L::get(py, i);
-  dual_math<P, TGV, GAP>(ub[i], ub[ixp], ub[iyp], vx0, vy0, vxx, vyx, vxy, vyy, pxv, pyv, qxx, qyy, qxy, sigma, ia0,
-                         ia1, t);
+  dual_math<P, TGV, GAP>(ub[i], ub[ixp], ub[iyp], vx0, vy0, vxx, vyx, vxy, vyy, pxv, pyv, qxx, qyy, qxy, sigma, w0,
+                         w1, t);
   if (TGV) {
     L::put(qxxp, i, qxx);
     L::put(qyyp, i, qyy);
@@ -902,17 +736,6 @@ __device__ __forceinline__ double vstep_pixel(const SliceDev& d, int x, int y, t
   return dabs2(pxi + dsx) + dabs2(pyi + dsy);
 }
 
-__device__ __forceinline__ bool slice_active(const SliceDev& d) { return gptr<const int>(d.ctl)[CTL_ACTIVE] != 0; }
-
-// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-// L2).  Give XCD x a contiguous range of logical work items, so that items
-// touching neighbouring memory (adjacent column groups, adjacent rows) share
-// one L2.  Bijective on [0, n).
-__device__ __forceinline__ int xcd_item(int b, int n) {
-  const int q = n >> 3, r = n & 7, x = b & 7, k = b >> 3;
-  return x * q + min(x, r) + k;
-}
-
 // ---------------------------------------------------------------------------
 // Denoising half-iterations.  Item = (slice, first row); rpi rows per item.
 // ---------------------------------------------------------------------------
@@ -936,7 +759,7 @@ __global__ __launch_bounds__(NT) void k_tv_dual(const SliceDev* sl, const int2* 
   for (int idx = threadIdx.x; idx < cnt; idx += NT) {
     const int yy = idx / W;
     const int x = idx - yy * W, y = ya + yy;
-    dual_pixel<P, P, false, GAP>(d, x, y, sigma, R(0), R(0), t);
+    dual_pixel<P, P, false, GAP>(d, x, y, sigma, R(0), ball_weight(R(1)), t);
     if (GAP) {
       const size_t i = size_t(y) * W + x;
       t[3] += dabs2(ub[i] - f[i]);
@@ -985,327 +808,6 @@ __global__ __launch_bounds__(NT) void k_tv_primal(const SliceDev* sl, const int2
   if (ya == 0 && threadIdx.x == 0) gptr<int>(d.ctl)[CTL_ITER] += 1;
 }
 
-// Temporally blocked ROF iterations: tb_k times TV_dual_p_kernel then
-// TV_primal_u_kernel (tgv_kernels.cuh:294-324,568-605) per launch, on a tile
-// held by the workgroup.  Block (bx, by) owns the interior [x0, x1) x [y0, y1)
-// and loads u, ubar, p (2 planes) and f on the interior grown by k pixels on
-// every side (clipped to the image).  Each iteration shrinks the region
-// where the values are exact by one pixel on each side that is not an image
-// border: the dual step at (x, y) needs ubar at x + 1 and y + 1 (forward
-// differences, none at the last column/row), the primal step p at x - 1 and
-// y - 1 (backward differences, none at the first).  After k iterations the
-// interior is exact and is written to the other copy of the state (src ->
-// dst), so that no block reads a halo that another block of the same launch
-// writes.  Each thread owns up to tv_block_own pixels of the tile for the
-// whole launch and keeps their u, f and p in registers (only the pixel
-// itself reads u and f, and its own p in the dual step); ubar and p, which
-// neighbours read, are the three LDS planes.  The per-pixel arithmetic is
-// that of k_tv_dual / k_tv_primal, in the same order, so the iterates equal
-// theirs bit for bit.
-constexpr int tv_block_own(size_t) { return 4; }  // (block_threads: 4 pixels per thread up to 4096)
-
-template <class P, int NT>
-__global__ __launch_bounds__(NT) void k_tv_block(const SliceDev* sl, int tx, int ty, int k, int dir) {
-  extern __shared__ char smem_raw[];
-  constexpr int J = tv_block_own(sizeof(P));
-  const SliceDev& d = sl[0];
-  if (!slice_active(d)) return;
-  using R = typename RealOf<P>::T;
-  const int W = d.W, H = d.H;
-  const int nbx = (W + tx - 1) / tx;
-  const int b = xcd_item(blockIdx.x, gridDim.x);  // neighbouring tiles on one XCD
-  const int by = b / nbx, bx = b - by * nbx;
-  const int x0 = bx * tx, x1 = min(W, x0 + tx), y0 = by * ty, y1 = min(H, y0 + ty);
-  const int xa = max(0, x0 - k), xb = min(W, x1 + k), ya = max(0, y0 - k), yb = min(H, y1 + k);
-  const int LW = xb - xa, LN = LW * (yb - ya);  // LN <= J * NT (block_fits)
-  P* sB = reinterpret_cast<P*>(smem_raw);
-  P* sX = sB + LN;
-  P* sY = sX + LN;
-  const size_t n = size_t(W) * H;
-  // the owned pixels e = threadIdx.x + j NT of the tile (x = -1: none)
-  P ru[J], rf[J], rpx[J], rpy[J];
-  int rx[J], ry[J];
-  {
-    const auto gu = gptr<const P>(dir ? d.u2 : d.u);
-    const auto gb = gptr<const P>(dir ? d.ub2 : d.ub);
-    const auto gp = gptr<const P>(dir ? d.p2 : d.p);
-    const auto gf = gptr<const P>(d.f);
-    const float rLW = 1.0f / float(LW);
-    P vb[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int e = threadIdx.x + j * NT;
-      rx[j] = -1;
-      ry[j] = -1;
-      if (e < LN) {
-        const int ly = qdiv(e, LW, rLW), lx = e - ly * LW;
-        rx[j] = xa + lx;
-        ry[j] = ya + ly;
-        const size_t gi = size_t(ry[j]) * W + rx[j];
-        ru[j] = gu[gi];
-        vb[j] = gb[gi];
-        rpx[j] = gp[gi];
-        rpy[j] = gp[gi + n];
-        rf[j] = gf[gi];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int e = threadIdx.x + j * NT;
-      if (e < LN) {
-        sB[e] = vb[j];
-        sX[e] = rpx[j];
-        sY[e] = rpy[j];
-      }
-    }
-  }
-  __syncthreads();
-  const R sigma = R(d.sigma), tau = R(d.tau), lambda = R(d.lambda), theta = R(d.theta);
-  int uxa = xa, uxb = xb, uya = ya, uyb = yb;  // where u, ubar are exact
-  for (int it = 0; it < k; ++it) {
-    // dual step where ubar and its forward neighbours are exact
-    const int pxa = uxa, pxb = uxb == W ? W : uxb - 1, pya = uya, pyb = uyb == H ? H : uyb - 1;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int x = rx[j], y = ry[j];
-      if (x >= pxa && x < pxb && y >= pya && y < pyb) {
-        const int l = threadIdx.x + j * NT;
-        const P c = sB[l], ex = sB[l + (x < W - 1)], ey = sB[l + ((y < H - 1) ? LW : 0)];
-        const P tx_ = ex - c, ty_ = ey - c;
-        const P ax = rpx[j] + sigma * tx_;
-        const P ay = rpy[j] + sigma * ty_;
-        const R pn = sqrt(abs2(ax) + abs2(ay));
-        const R sp = rcp(fmax(R(1), pn));
-        rpx[j] = ax * sp;
-        rpy[j] = ay * sp;
-        sX[l] = rpx[j];
-        sY[l] = rpy[j];
-      }
-    }
-    __syncthreads();
-    // primal step where p and its backward neighbours are exact
-    uxa = pxa == 0 ? 0 : pxa + 1;
-    uxb = pxb;
-    uya = pya == 0 ? 0 : pya + 1;
-    uyb = pyb;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int x = rx[j], y = ry[j];
-      if (x >= uxa && x < uxb && y >= uya && y < uyb) {
-        const int l = threadIdx.x + j * NT;
-        const P cx = rpx[j], mx = sX[x > 0 ? l - 1 : l];
-        const P dx = (x < W - 1) ? cx - mx : -mx;
-        const P cy = rpy[j], my = sY[y > 0 ? l - LW : l];
-        const P dy = (y < H - 1) ? cy - my : -my;
-        const P div = (x > 0 ? dx : cx) + (y > 0 ? dy : cy);
-        const P uo = ru[j];
-        P un = uo + tau * fmadd(lambda, rf[j], div);
-        un = un * rcp(R(1) + tau * lambda);
-        ru[j] = un;
-        sB[l] = (R(1) + theta) * un - theta * uo;
-      }
-    }
-    __syncthreads();
-  }
-  const auto ou = gptr<P>(dir ? d.u : d.u2);
-  const auto ob = gptr<P>(dir ? d.ub : d.ub2);
-  const auto op = gptr<P>(dir ? d.p : d.p2);
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int x = rx[j], y = ry[j];
-    if (x >= x0 && x < x1 && y >= y0 && y < y1) {
-      const int l = threadIdx.x + j * NT;
-      const size_t gi = size_t(y) * W + x;
-      ou[gi] = ru[j];
-      ob[gi] = sB[l];
-      op[gi] = rpx[j];
-      op[gi + n] = rpy[j];
-    }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) gptr<int>(d.ctl)[CTL_ITER] += k;
-}
-
-// The value a dual field holds after a store to its storage type S and a
-// load back (S = P: itself; fp16 storage: rounded to half).
-template <class P, class S>
-__device__ __forceinline__ P storage_round(P v) {
-  S s[1];
-  Ld<P, S>::put(s, 0, v);
-  return Ld<P, S>::get(s, 0);
-}
-
-// Temporally blocked TGV denoising: tb_k times the primal step
-// (TV_primal_u_kernel + TGV_primal_v_kernel) then the dual step
-// (TGV_dual_p_kernel + TGV_dual_q_kernel) per launch, in the reference's
-// order (tgvoptimizer.cu:119-135; tgv_kernels.cuh:225-292,568-605,647-686),
-// on a tile.  Block (bx, by) owns the interior [x0, x1) x [y0, y1) and loads
-// u, v (2 planes), p (2), q (3) and f on the interior grown by k pixels on
-// every side (clipped to the image).  The primal step at (x, y) needs p, q at
-// x - 1 and y - 1 (backward differences, none at the first column / row), the
-// dual step ubar, vbar at x + 1 and y + 1 (forward differences, none at the
-// last): the region where the values are exact shrinks by one pixel per step
-// on each side that is not an image border, and after k iterations the
-// interior is exact.  It is written with ubar and vbar to the other copy of
-// the state (src -> dst).  Each thread owns up to tgv_block_own pixels of the
-// tile for the whole launch and keeps their u, v and f, which only the
-// pixel itself reads, in registers; ubar, vbar, p and q, which neighbours
-// read, live in LDS (two pixels per thread for 16-byte values, in
-// workgroups of at most 512 threads, whose registers would not hold more).
-// The per-pixel arithmetic
-// is that of k_tgv_primal /
-// k_tgv_dual in the same order, and the duals are rounded to their storage
-// type after every dual step (as a store and a load would round them), so
-// the iterates equal theirs bit for bit.
-constexpr int tgv_block_own(size_t value_bytes) { return value_bytes > 8 ? 2 : 3; }
-
-template <class P, class S, int NT>
-__global__ __launch_bounds__(NT) void k_tgv_block(const SliceDev* sl, int tx, int ty, int k, int dir) {
-  extern __shared__ char smem_raw[];
-  constexpr int J = tgv_block_own(sizeof(P));
-  using R = typename RealOf<P>::T;
-  using L = Ld<P, S>;
-  const SliceDev& d = sl[0];
-  if (!slice_active(d)) return;
-  const int W = d.W, H = d.H;
-  const int nbx = (W + tx - 1) / tx;
-  const int b = xcd_item(blockIdx.x, gridDim.x);  // neighbouring tiles on one XCD
-  const int by = b / nbx, bx = b - by * nbx;
-  const int x0 = bx * tx, x1 = min(W, x0 + tx), y0 = by * ty, y1 = min(H, y0 + ty);
-  const int xa = max(0, x0 - k), xb = min(W, x1 + k), ya = max(0, y0 - k), yb = min(H, y1 + k);
-  const int LW = xb - xa, LN = LW * (yb - ya);  // LN <= J * NT (block_fits)
-  P* sUB = reinterpret_cast<P*>(smem_raw);
-  P* sVBX = sUB + LN;
-  P* sVBY = sVBX + LN;
-  P* sPX = sVBY + LN;
-  P* sPY = sPX + LN;
-  P* sQXX = sPY + LN;
-  P* sQYY = sQXX + LN;
-  P* sQXY = sQYY + LN;
-  const size_t n = size_t(W) * H;
-  // the owned pixels e = threadIdx.x + j NT of the tile (x = -1: none)
-  P ru[J], rvx[J], rvy[J], rf[J];
-  int rx[J], ry[J];
-  {
-    const auto gu = gptr<const P>(dir ? d.u2 : d.u);
-    const auto gv = gptr<const P>(dir ? d.v2 : d.v);
-    const auto gp = gptr<const S>(dir ? d.p2 : d.p);
-    const auto gq = gptr<const S>(dir ? d.q2 : d.q);
-    const auto gf = gptr<const P>(d.f);
-    const float rLW = 1.0f / float(LW);
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int e = threadIdx.x + j * NT;
-      rx[j] = -1;
-      ry[j] = -1;
-      if (e < LN) {
-        const int ly = qdiv(e, LW, rLW), lx = e - ly * LW;
-        rx[j] = xa + lx;
-        ry[j] = ya + ly;
-        const size_t gi = size_t(ry[j]) * W + rx[j];
-        ru[j] = gu[gi];
-        rvx[j] = gv[gi];
-        rvy[j] = gv[gi + n];
-        rf[j] = gf[gi];
-        sPX[e] = L::get(gp, gi);
-        sPY[e] = L::get(gp, gi + n);
-        sQXX[e] = L::get(gq, gi);
-        sQYY[e] = L::get(gq, gi + n);
-        sQXY[e] = L::get(gq, gi + 2 * n);
-      }
-    }
-  }
-  __syncthreads();
-  const R sigma = R(d.sigma), tau = R(d.tau), lambda = R(d.lambda), theta = R(d.theta);
-  const R ia0 = rcp(R(d.alpha0)), ia1 = rcp(R(d.alpha1));
-  // backward differences dmx / dmy on the tile
-  auto bdx = [&](const P* a, int l, int x) {
-    const P c = a[l], m = a[x > 0 ? l - 1 : l];
-    const P dd = (x < W - 1) ? c - m : -m;
-    return x > 0 ? dd : c;
-  };
-  auto bdy = [&](const P* a, int l, int y) {
-    const P c = a[l], m = a[y > 0 ? l - LW : l];
-    const P dd = (y < H - 1) ? c - m : -m;
-    return y > 0 ? dd : c;
-  };
-  int pxa = xa, pxb = xb, pya = ya, pyb = yb;  // where p, q are exact
-  for (int it = 0; it < k; ++it) {
-    // primal step where p, q and their backward neighbours are exact
-    const int uxa = pxa == 0 ? 0 : pxa + 1, uxb = pxb, uya = pya == 0 ? 0 : pya + 1, uyb = pyb;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int x = rx[j], y = ry[j];
-      if (x >= uxa && x < uxb && y >= uya && y < uyb) {
-        const int l = threadIdx.x + j * NT;
-        const P uo = ru[j];
-        const P div = bdx(sPX, l, x) + bdy(sPY, l, y);
-        P un = uo + tau * fmadd(lambda, rf[j], div);
-        un = un * rcp(R(1) + tau * lambda);
-        ru[j] = un;
-        sUB[l] = (R(1) + theta) * un - theta * uo;
-        const P dsx = bdx(sQXX, l, x) + bdy(sQXY, l, y);
-        const P dsy = bdy(sQYY, l, y) + bdx(sQXY, l, x);
-        const P ox = rvx[j], oy = rvy[j];
-        const P nx = ox + tau * (dsx + sPX[l]);
-        const P ny = oy + tau * (dsy + sPY[l]);
-        rvx[j] = nx;
-        rvy[j] = ny;
-        sVBX[l] = (R(1) + theta) * nx - theta * ox;
-        sVBY[l] = (R(1) + theta) * ny - theta * oy;
-      }
-    }
-    __syncthreads();
-    // dual step where ubar, vbar and their forward neighbours are exact
-    pxa = uxa;
-    pxb = uxb == W ? W : uxb - 1;
-    pya = uya;
-    pyb = uyb == H ? H : uyb - 1;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int x = rx[j], y = ry[j];
-      if (x >= pxa && x < pxb && y >= pya && y < pyb) {
-        const int l = threadIdx.x + j * NT;
-        const int lx = l + (x < W - 1), ly = l + ((y < H - 1) ? LW : 0);
-        P px = sPX[l], py = sPY[l], qxx = sQXX[l], qyy = sQYY[l], qxy = sQXY[l];
-        dual_math<P, true, false>(sUB[l], sUB[lx], sUB[ly], sVBX[l], sVBY[l], sVBX[lx], sVBY[lx], sVBX[ly], sVBY[ly],
-                                  px, py, qxx, qyy, qxy, sigma, ia0, ia1, nullptr);
-        sPX[l] = storage_round<P, S>(px);
-        sPY[l] = storage_round<P, S>(py);
-        sQXX[l] = storage_round<P, S>(qxx);
-        sQYY[l] = storage_round<P, S>(qyy);
-        sQXY[l] = storage_round<P, S>(qxy);
-      }
-    }
-    __syncthreads();
-  }
-  const auto ou = gptr<P>(dir ? d.u : d.u2);
-  const auto oub = gptr<P>(dir ? d.ub : d.ub2);
-  const auto ov = gptr<P>(dir ? d.v : d.v2);
-  const auto ovb = gptr<P>(dir ? d.vb : d.vb2);
-  const auto op = gptr<S>(dir ? d.p : d.p2);
-  const auto oq = gptr<S>(dir ? d.q : d.q2);
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int x = rx[j], y = ry[j];
-    if (x >= x0 && x < x1 && y >= y0 && y < y1) {
-      const int l = threadIdx.x + j * NT;
-      const size_t gi = size_t(y) * W + x;
-      ou[gi] = ru[j];
-      oub[gi] = sUB[l];
-      ov[gi] = rvx[j];
-      ov[gi + n] = rvy[j];
-      ovb[gi] = sVBX[l];
-      ovb[gi + n] = sVBY[l];
-      L::put(op, gi, sPX[l]);
-      L::put(op, gi + n, sPY[l]);
-      L::put(oq, gi, sQXX[l]);
-      L::put(oq, gi + n, sQYY[l]);
-      L::put(oq, gi + 2 * n, sQXY[l]);
-    }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) gptr<int>(d.ctl)[CTL_ITER] += k;
-}
-
 // TGV denoising primal half (tgvoptimizer.cu:119-127): TV_primal_u_kernel
 // then TGV_primal_v_kernel at every pixel.
 template <class P, class S, int NT>
@@ -1350,7 +852,7 @@ __global__ __launch_bounds__(NT) void k_tgv_dual(const SliceDev* sl, const int2*
   using R = typename RealOf<P>::T;
   const int W = d.W, H = d.H;
   const int ya = it.y, yb = min(H, ya + rpi);
-  const R sigma = R(d.sigma), a0 = R(d.alpha0), a1 = R(d.alpha1);
+  const R sigma = R(d.sigma), w0 = ball_weight(R(d.alpha0)), w1 = ball_weight(R(d.alpha1));
   const auto ub = gptr<const P>(d.ub);
   const auto f = gptr<const P>(d.f);
   double t[kGapTerms] = {0};
@@ -1358,7 +860,7 @@ __global__ __launch_bounds__(NT) void k_tgv_dual(const SliceDev* sl, const int2*
   for (int idx = threadIdx.x; idx < cnt; idx += NT) {
     const int yy = idx / W;
     const int x = idx - yy * W, y = ya + yy;
-    dual_pixel<P, S, true, GAP>(d, x, y, sigma, rcp(a0), rcp(a1), t);
+    dual_pixel<P, S, true, GAP>(d, x, y, sigma, w0, w1, t);
     if (GAP) {
       const size_t i = size_t(y) * W + x;
       t[3] += dabs2(ub[i] - f[i]);
@@ -1388,7 +890,7 @@ __global__ __launch_bounds__(NT) void k_tgv_dual2(const SliceDev* sl, const int2
   const int W = d.W, H = d.H;
   const size_t n = size_t(W) * H;
   const int ya = it.y, yb = min(H, ya + rpi);
-  const R sigma = R(d.sigma), ia0 = rcp(R(d.alpha0)), ia1 = rcp(R(d.alpha1));
+  const R sigma = R(d.sigma), w0 = ball_weight(R(d.alpha0)), w1 = ball_weight(R(d.alpha1));
   const auto ub = gptr<const P>(d.ub);
   const auto ubp = gptr<const Pair<P>>(d.ub);
   const auto vbx = gptr<const P>(d.vb);
@@ -1417,10 +919,10 @@ __global__ __launch_bounds__(NT) void k_tgv_dual2(const SliceDev* sl, const int2
     P qxxb = L::get(&qs[0].b, 0), qyyb = L::get(&qs[1].b, 0), qxyb = L::get(&qs[2].b, 0);
     // pixel x (never the last column), then x + 1
     dual_math<P, true, GAP>(u0.a, u0.b, bottom ? u0.a : ud.a, vx.a, vy.a, vx.b, vy.b, bottom ? vx.a : vxd.a,
-                            bottom ? vy.a : vyd.a, pxa, pya, qxxa, qyya, qxya, sigma, ia0, ia1, t);
+                            bottom ? vy.a : vyd.a, pxa, pya, qxxa, qyya, qxya, sigma, w0, w1, t);
     dual_math<P, true, GAP>(u0.b, last ? u0.b : u2, bottom ? u0.b : ud.b, vx.b, vy.b, last ? vx.b : vx2,
                             last ? vy.b : vy2, bottom ? vx.b : vxd.b, bottom ? vy.b : vyd.b, pxb, pyb, qxxb, qyyb,
-                            qxyb, sigma, ia0, ia1, t);
+                            qxyb, sigma, w0, w1, t);
     L::put(&ps[0].a, 0, pxa);
     L::put(&ps[0].b, 0, pxb);
     L::put(&ps[1].a, 0, pya);
@@ -1581,13 +1083,13 @@ __device__ __forceinline__ void dual_workgroup(const SliceDev& d, int nd, double
   const int pa = min(WH, b * chunk), pe = min(WH, pa + chunk);
   const int k = gptr<int>(d.ctl)[CTL_ITER];
   const R sigma = R(d.sigma);
-  const R ia0 = rcp(sched_alpha<R>(d, d.alpha0, d.alpha0_end, k));
-  const R ia1 = rcp(sched_alpha<R>(d, d.alpha1, d.alpha1_end, k));
+  const R w0 = ball_weight(sched_alpha<R>(d, d.alpha0, d.alpha0_end, k));
+  const R w1 = ball_weight(sched_alpha<R>(d, d.alpha1, d.alpha1_end, k));
   const float rW = 1.0f / float(W);
   double t[kGapTerms] = {0};
   for (int i = pa + threadIdx.x; i < pe; i += NT) {
     const int y = qdiv(i, W, rW), x = i - y * W;
-    dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, ia0, ia1, t);
+    dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, w0, w1, t);
   }
   if (GAP) block_sum<3, NT>(reinterpret_cast<double(&)[3]>(t), part + size_t(b) * kGapTerms);
 }
@@ -1662,8 +1164,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GAP ? 5 : 1)
     const R sigma = R(d.sigma);
     const R a0 = sched_alpha<R>(d, d.alpha0, d.alpha0_end, k);
     const R a1 = sched_alpha<R>(d, d.alpha1, d.alpha1_end, k);
-    const R ia0 = rcp(a0), ia1 = rcp(a1);
-    for (int x = xa + threadIdx.x; x < xe; x += NT) dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, ia0, ia1, t);
+    const R w0 = ball_weight(a0), w1 = ball_weight(a1);
+    for (int x = xa + threadIdx.x; x < xe; x += NT) dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, w0, w1, t);
   }
   if (NF > 0) {
     s_tw.store(L.tw, W);
@@ -2646,61 +2148,6 @@ static void with_fft_len(int n, Fn&& fn) {
   fn(std::integral_constant<int, 0>{});
 }
 
-size_t block_lds(int kind, int dtype, int tx, int ty, int k) {
-  const size_t e = dtype == DT_F32 ? 4 : (dtype == DT_C128 ? 16 : 8);
-  const size_t planes = kind == K_TGV ? 8 : 3;  // TGV: ubar, vbar, p, q; ROF: ubar, p
-  return planes * size_t(tx + 2 * k) * size_t(ty + 2 * k) * e;
-}
-
-// Workgroup size of a blocked launch: a few owned pixels per thread of the
-// loaded tile (ROF: up to 4 below 4096 pixels, TGV: one to tgv_block_own),
-// 256 to 1024 threads.
-static int block_threads(int kind, int dtype, int tx, int ty, int k) {
-  const int px = (tx + 2 * k) * (ty + 2 * k);
-  if (kind == K_TGV) return px >= 1024 && dtype != DT_C128 ? 1024 : px >= 384 ? 512 : 256;
-  return px > 2048 ? 1024 : px > 1024 ? 512 : 256;
-}
-
-bool block_fits(int kind, int dtype, int tx, int ty, int k, size_t lds_limit) {
-  if (tx <= 0 || ty <= 0 || k <= 0) return false;
-  const int px = (tx + 2 * k) * (ty + 2 * k);
-  // every tile pixel owned by a thread (TGV: tgv_block_own per thread at most)
-  const size_t e = dtype == DT_F32 ? 4 : (dtype == DT_C128 ? 16 : 8);
-  if (kind == K_TGV && px > tgv_block_own(e) * block_threads(kind, dtype, tx, ty, k)) return false;
-  // ROF: likewise, tv_block_own pixels per thread at most
-  if (kind != K_TGV && px > tv_block_own(e) * block_threads(kind, dtype, tx, ty, k)) return false;
-  return block_lds(kind, dtype, tx, ty, k) <= lds_limit;
-}
-
-void run_block(const Launch& L, int kind, int dtype, bool fp16, int dir) {
-  const int tx = L.tb_x, ty = L.tb_y, k = L.tb_k;
-  const size_t lds = block_lds(kind, dtype, tx, ty, k);
-  const int grid = ((L.tb_w + tx - 1) / tx) * ((L.tb_h + ty - 1) / ty);
-  auto launch = [&](auto nt) {
-    constexpr int NT = decltype(nt)::value;
-#define PDT_BLOCK(P, S)                                                                                             \
-  if (kind == K_TGV) hipLaunchKernelGGL((k_tgv_block<P, S, NT>), dim3(grid), dim3(NT), lds, L.stream, L.sl, tx, ty, k, dir); \
-  else hipLaunchKernelGGL((k_tv_block<P, NT>), dim3(grid), dim3(NT), lds, L.stream, L.sl, tx, ty, k, dir)
-    switch (dtype) {
-      case DT_F32:
-        if (fp16 && kind == K_TGV) hipLaunchKernelGGL((k_tgv_block<float, _Float16, NT>), dim3(grid), dim3(NT), lds, L.stream, L.sl, tx, ty, k, dir);
-        else PDT_BLOCK(float, float);
-        break;
-      case DT_C64:
-        if (fp16 && kind == K_TGV) hipLaunchKernelGGL((k_tgv_block<Cx<float>, Cx<_Float16>, NT>), dim3(grid), dim3(NT), lds, L.stream, L.sl, tx, ty, k, dir);
-        else PDT_BLOCK(Cx<float>, Cx<float>);
-        break;
-      case DT_F64: PDT_BLOCK(double, double); break;
-      case DT_C128: PDT_BLOCK(Cx<double>, Cx<double>); break;
-    }
-#undef PDT_BLOCK
-  };
-  const int nt = block_threads(kind, dtype, tx, ty, k);
-  if (nt == 1024) launch(std::integral_constant<int, 1024>{});
-  else if (nt == 512) launch(std::integral_constant<int, 512>{});
-  else launch(std::integral_constant<int, 256>{});
-}
-
 bool fft_len_compiled(int dtype, int n) {
   if (dtype != DT_C64 && dtype != DT_F32) return false;
   for (int m : kFftLengths)
@@ -2949,26 +2396,6 @@ static bool set_lds_attrs(int b) {
     set((const void*)&k_cols<R, CM_FWD, false, NC, NF>);
     set((const void*)&k_cols<R, CM_ADJ, false, NC, NF>);
   };
-  set((const void*)&k_tv_block<R, 256>);
-  set((const void*)&k_tv_block<Cx<R>, 256>);
-  set((const void*)&k_tv_block<R, 512>);
-  set((const void*)&k_tv_block<Cx<R>, 512>);
-  set((const void*)&k_tv_block<R, 1024>);
-  set((const void*)&k_tv_block<Cx<R>, 1024>);
-  set((const void*)&k_tgv_block<R, R, 256>);
-  set((const void*)&k_tgv_block<Cx<R>, Cx<R>, 256>);
-  set((const void*)&k_tgv_block<R, R, 512>);
-  set((const void*)&k_tgv_block<Cx<R>, Cx<R>, 512>);
-  set((const void*)&k_tgv_block<R, R, 1024>);
-  set((const void*)&k_tgv_block<Cx<R>, Cx<R>, 1024>);
-  if constexpr (std::is_same<R, float>::value) {
-    set((const void*)&k_tgv_block<float, _Float16, 256>);
-    set((const void*)&k_tgv_block<Cx<float>, Cx<_Float16>, 256>);
-    set((const void*)&k_tgv_block<float, _Float16, 512>);
-    set((const void*)&k_tgv_block<Cx<float>, Cx<_Float16>, 512>);
-    set((const void*)&k_tgv_block<float, _Float16, 1024>);
-    set((const void*)&k_tgv_block<Cx<float>, Cx<_Float16>, 1024>);
-  }
   with_fft_len<R>(0, one);
   for (int n : kFftLengths)
     if (std::is_same<R, float>::value) with_fft_len<R>(n, one);

@@ -69,9 +69,9 @@ struct Launch {
   // the LDS of a CU (the autotuner's waves-per-CU axis)
   int wpc[4] = {0, 0, 0, 0};
   // temporally blocked denoising launches (one dense ROF or TGV slice):
-  // interior tile tb_x x tb_y pixels, tb_k iterations per launch (0: off)
+  // interior tile tb_x x tb_y pixels (block_shape), tb_k iterations per
+  // launch (0: off)
   int tb_x = 0, tb_y = 0, tb_k = 0;
-  int tb_w = 0, tb_h = 0;  // the slice's image size (grid of tiles)
 };
 enum { WPC_FWD = 0, WPC_COLS = 1, WPC_ADJ = 2, WPC_DEN = 3 };
 
@@ -97,15 +97,26 @@ void run_stage(const Launch& L, int kind, int dtype, bool fp16, bool gap, int st
 // the gap-evaluation variants (partial sums where the three passes put them).
 // The first iteration of a solve starts from stages 0 and 1 instead of 0.
 void run_pair_stage(const Launch& L, int kind, int dtype, int which, bool gap);
-// tb_k ROF or TGV (kind) iterations of a single dense slice in one launch
-// (tiles held in LDS with a tb_k-pixel halo), reading the state (ROF: u,
-// ubar, p; TGV: u, v, p, q) and writing its second copy with ubar (and vbar)
-// (dir = 0) or the reverse (dir = 1); fp16: TGV duals stored as half.
-void run_block(const Launch& L, int kind, int dtype, bool fp16, int dir);
-// LDS bytes of that launch, and whether a tile shape fits (the LDS a
-// workgroup may take, and for TGV the pixels its threads can own).
-size_t block_lds(int kind, int dtype, int tx, int ty, int k);
-bool block_fits(int kind, int dtype, int tx, int ty, int k, size_t lds_limit);
+// The launch of k blocked ROF or TGV (kind) iterations on a W x H slice with
+// interior tiles of tx x ty pixels: the exact region of a workgroup (at most
+// 64 columns and the rows its waves hold; tiles are cut to fit), its waves and
+// the number of workgroups (0: the halo leaves no interior).
+struct BlockShape {
+  int rx = 0, ry = 0, waves = 0, grid = 0;
+};
+BlockShape block_shape(int kind, int dtype, int W, int H, int tx, int ty, int k);
+// The tile (x, y, iterations) of a W x H slice without a tuned or forced one,
+// and the ranges it is chosen from (iterations per launch, waves per
+// workgroup), which the autotuner times.
+void block_choose(int kind, int dtype, bool fp16, int W, int H, int tile[3]);
+constexpr int kBlockIterations[] = {3, 4, 5, 6, 8, 10, 12, 16, 20};
+constexpr int kBlockWaves[] = {4, 8, 12, 16};
+constexpr int kBlockRows = 4;  // rows per wave
+// Those k iterations of the single dense slice of L (d: its descriptor, on
+// the host), reading the state (ROF: u, ubar, p; TGV: u, v, p, q) and writing
+// its second copy (dir = 0) or the reverse (dir = 1); fp16: TGV duals stored
+// as half.
+void run_block(const Launch& L, const SliceDev& d, int kind, int dtype, bool fp16, int dir, int k);
 // Gap evaluation from the partial sums of the last iteration (one block/slice).
 void run_gap_reduce(const Launch& L, int kind, int dtype);
 // Operator application in operator mode (op_in -> op_out of every slice).

@@ -262,9 +262,13 @@ PDT_API int pdt_autotune(pdt_solver** solvers, int count, int reps, pdt_tiles* o
  * uses it. */
 PDT_API int pdt_set_tiles(pdt_solver** solvers, int count, const pdt_tiles* tiles);
 
-/* NEW: solve many configured solvers (same kind and dtype) together, with one
- * persistent work-list launch per half-iteration for the whole batch.  Each
- * solver keeps its own parameters, sizes, coils and stopping. */
+/* NEW: solve many configured solvers (same kind and dtype) together: with one
+ * persistent work-list launch per half-iteration for the whole batch, or, for
+ * operator solvers of large slices or many sizes, as concurrent single solves
+ * (pdt_solve_concurrent), whichever a rule on the sizes takes to be faster
+ * (batches with tuned or set tiles, without graphs or verbose: always the
+ * work lists).  Each solver keeps its own parameters, sizes, coils and
+ * stopping. */
 PDT_API int pdt_batch_solve(pdt_solver** solvers, int count, int verbose);
 
 /* NEW (no counterpart in the reference, which solves one problem per call,

@@ -804,6 +804,18 @@ void prepare_op_data(pdt_solver* s) {
   s->data_dirty = false;
 }
 
+// Tile-cache key of operator solvers run together.
+TuneKey mri_key(const std::vector<pdt_solver*>& sv) {
+  TuneKey k{sv[0]->kind, sv[0]->dtype == PDT_C128 ? DT_C128 : DT_C64, 0, sv[0]->H, 0, 1, 1, int(sv.size())};
+  for (auto* s : sv) {
+    k.W = std::max(k.W, s->W);
+    k.Hk = std::max(k.Hk, s->op->Hk);
+    k.C = std::max(k.C, s->op->C);
+    k.nc = std::max(k.nc, s->op->ncols);
+  }
+  return k;
+}
+
 // ---------------------------------------------------------------------------
 // The engine: one or many slices, persistent work lists, graph-replayed chunks
 // ---------------------------------------------------------------------------
@@ -885,7 +897,7 @@ struct Engine {
         maxC = std::max(maxC, s->op->C);
         maxNc = std::max(maxNc, s->op->ncols);
       }
-      key = TuneKey{kind, dt, maxW, sv[0]->H, maxHk, maxC, maxNc, ns};
+      key = mri_key(sv);
       TuneVal tv = tune_lookup(key);
       for (int i = 0; i < 4; ++i) L.wpc[i] = force_wpc[i] >= 0 ? force_wpc[i] : tv.wpc[i];
       unpaired = force_unpaired >= 0 ? force_unpaired != 0 : tv.unpaired != 0;
@@ -1617,33 +1629,110 @@ void check_batch(const std::vector<pdt_solver*>& sv) {
   }
 }
 
+// Runs solve_one on every solver, `streams` at a time: the calling thread and
+// streams - 1 more take the next solver in order; the first failure stops the
+// others from taking more and is thrown here.
+template <class F>
+void solve_pool(const std::vector<pdt_solver*>& sv, int streams, F&& solve_one) {
+  const int count = (int)sv.size();
+  int dev = 0;
+  HIPC(hipGetDevice(&dev));
+  std::atomic<int> next{0};
+  std::atomic<bool> failed{false};
+  std::mutex mu;
+  int err_code = PDT_OK;
+  std::string err_msg;
+  auto work = [&] {
+    const int rc = guard([&] {
+      HIPC(hipSetDevice(dev));
+      for (;;) {
+        if (failed.load()) return;
+        const int i = next.fetch_add(1);
+        if (i >= count) return;
+        solve_one(sv[i]);
+      }
+    });
+    if (rc != PDT_OK) {
+      failed.store(true);
+      std::lock_guard<std::mutex> lk(mu);
+      if (err_code == PDT_OK) {
+        err_code = rc;
+        err_msg = g_err;
+      }
+    }
+  };
+  std::vector<std::thread> pool;
+  for (int t = 1; t < std::min(streams, count); ++t) pool.emplace_back(work);
+  work();
+  for (auto& t : pool) t.join();
+  if (err_code != PDT_OK) fail(err_code, err_msg);
+}
+
+// One prepared solver alone, on its cached engine: its work lists and
+// instantiated graphs stay valid while nothing they depend on changed (a
+// replaced engine is released, and the new one built, under the set-up lock).
+void solve_single(pdt_solver* s, int verbose) {
+  std::shared_ptr<Engine> cached;
+  {
+    SetupLock lk(g_setup_mu);
+    Engine probe;
+    probe.sv = {s};
+    probe.plan_only = true;
+    probe.build();
+    cached = std::static_pointer_cast<Engine>(s->engine);
+    if (!cached || cached->sig != probe.sig) {
+      cached.reset();
+      s->engine.reset();
+      auto e = std::make_shared<Engine>();
+      e->sv = {s};
+      e->build();
+      s->engine = e;
+      cached = e;
+    }
+  }
+  cached->run(verbose);
+}
+
+// Whether a batch of prepared operator solvers is faster as single solves on
+// kBatchStreams streams than as one work-list launch per pass and group of
+// equal transform lengths.  A group's launches follow one another, each with
+// its own tail, and stream every slice through DRAM; single solves overlap,
+// run paired iterations and keep fewer slices in the caches, but pay a chunk's
+// start per slice.  Measured per 100 iterations (n slices in G groups, X
+// million sensitivities on the image windows): batched about 2.2 G + 0.1 n +
+// 1.5 X ms, single 0.65 n + 0.85 X ms, equal at n = 4 G + 1.2 X.  Eight slices
+// of 320 x 320, 15 coils: 21.0 against 15.5 ms, of 64 x 64, 8 coils: 3.6
+// against 7.5; eight mixed slices in four groups: 29.1 against 17.9.  A batch
+// whose tiles were tuned or set keeps the launches they were chosen for, as do
+// direct launches (no graphs) and verbose solves.
+constexpr int kBatchStreams = 4;
+bool batch_as_singles(const std::vector<pdt_solver*>& sv, int verbose) {
+  if (!sv[0]->is_op() || verbose || sv[0]->prm.use_graph == 0 || tune_has(mri_key(sv))) return false;
+  std::map<std::pair<int, int>, int> groups;
+  double x = 0;
+  for (auto* s : sv) {
+    groups[{s->op->W, s->op->Hk}]++;
+    x += 1e-6 * double(s->op->C) * s->W * s->H;
+  }
+  return double(sv.size()) < 4.0 * double(groups.size()) + 1.2 * x;
+}
+
 void solve_many(std::vector<pdt_solver*>& sv, int verbose) {
   check_batch(sv);
   for (auto* s : sv) prepare_solve(s, verbose);
   if (sv.size() == 1) {
-    // reuse the engine of the previous solve when nothing it depends on
-    // changed: its work lists and instantiated graphs stay valid (a replaced
-    // engine is released, and the new one built, under the set-up lock)
-    pdt_solver* s = sv[0];
-    std::shared_ptr<Engine> cached;
-    {
-      SetupLock lk(g_setup_mu);
-      Engine probe;
-      probe.sv = sv;
-      probe.plan_only = true;
-      probe.build();
-      cached = std::static_pointer_cast<Engine>(s->engine);
-      if (!cached || cached->sig != probe.sig) {
-        cached.reset();
-        s->engine.reset();
-        auto e = std::make_shared<Engine>();
-        e->sv = sv;
-        e->build();
-        s->engine = e;
-        cached = e;
-      }
-    }
-    cached->run(verbose);
+    solve_single(sv[0], verbose);
+    return;
+  }
+  if (batch_as_singles(sv, verbose)) {
+    const auto t0 = std::chrono::steady_clock::now();
+    auto since = [&] { return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count(); };
+    solve_pool(sv, kBatchStreams, [&](pdt_solver* s) {
+      solve_single(s, verbose);
+      s->stats.ms_to_stop = since();
+    });
+    const double ms = since();
+    for (auto* s : sv) s->stats.ms = ms;  // the loop's time, as of one set of launches
     return;
   }
   auto e = std::make_unique<Engine>();
@@ -2474,41 +2563,10 @@ int pdt_solve_concurrent(pdt_solver** solvers, int count, int streams, int verbo
       for (int j = 0; j < i; ++j)
         if (v[j] == v[i]) fail(PDT_ERR_ARG, "a solver appears twice in the batch");
     }
-    // Workers (the calling thread and streams - 1 more) take the next
-    // unsolved solver in order and solve it alone on its own stream; the
-    // first failure stops the others from taking more and is reported here.
-    int dev = 0;
-    HIPC(hipGetDevice(&dev));
-    std::atomic<int> next{0};
-    std::atomic<bool> failed{false};
-    std::mutex mu;
-    int err_code = PDT_OK;
-    std::string err_msg;
-    auto work = [&] {
-      const int rc = guard([&] {
-        HIPC(hipSetDevice(dev));
-        for (;;) {
-          if (failed.load()) return;
-          const int i = next.fetch_add(1);
-          if (i >= count) return;
-          std::vector<pdt_solver*> one{v[i]};
-          solve_many(one, verbose);
-        }
-      });
-      if (rc != PDT_OK) {
-        failed.store(true);
-        std::lock_guard<std::mutex> lk(mu);
-        if (err_code == PDT_OK) {
-          err_code = rc;
-          err_msg = g_err;
-        }
-      }
-    };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < std::min(streams, count); ++t) pool.emplace_back(work);
-    work();
-    for (auto& t : pool) t.join();
-    if (err_code != PDT_OK) fail(err_code, err_msg);
+    solve_pool(v, streams, [&](pdt_solver* s) {
+      std::vector<pdt_solver*> one{s};
+      solve_many(one, verbose);
+    });
   });
 }
 

@@ -81,6 +81,12 @@ TuneVal tune_lookup(const TuneKey& k) {
   return it == g_cache.end() ? TuneVal{} : it->second;
 }
 
+bool tune_has(const TuneKey& k) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  load_locked();
+  return g_cache.count(k) != 0;
+}
+
 void tune_store(const TuneKey& k, const TuneVal& v) {
   std::lock_guard<std::mutex> lk(g_mu);
   load_locked();

@@ -30,6 +30,8 @@ struct TuneVal {
 };
 
 TuneVal tune_lookup(const TuneKey& k);
+// Whether a choice is stored for k.
+bool tune_has(const TuneKey& k);
 void tune_store(const TuneKey& k, const TuneVal& v);
 
 }  // namespace pdt

@@ -305,8 +305,9 @@ def batch_profile(optimizers, reps: int = 20) -> list:
 
 
 def batch_solve(optimizers, verbose: bool = False) -> None:
-    """Solves configured optimizers of one class together, one persistent
-    work-list launch per half-iteration for the whole batch."""
+    """Solves configured optimizers of one class together: one persistent
+    work-list launch per half-iteration for the whole batch, or concurrent
+    single solves where those are faster (large slices, many sizes)."""
     if not optimizers:
         return
     for o in optimizers:

@@ -26,17 +26,6 @@ __device__ __forceinline__ float sel(bool c, float a, float b) { return c ? a : 
 __device__ __forceinline__ double sel(bool c, double a, double b) { return c ? a : b; }
 template <class R> __device__ __forceinline__ Cx<R> sel(bool c, Cx<R> a, Cx<R> b) { return csel(c, a, b); }
 
-// Workgroup barrier with its own wait for the wave's LDS accesses.  (At the
-// head of a loop whose last LDS store is at its end, the compiler drops the
-// wait of __syncthreads, which it finds satisfied on the way into the loop:
-// read in this build's assembly, where the barrier let a wave read the edge
-// row of the iteration before.)
-__device__ __forceinline__ void wg_barrier() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#endif
-}
-
 // A value as a store and a load would leave it: the empty register constraint
 // keeps the compiler from fusing the product that formed it with its use in
 // the next step (the one-iteration kernels, with memory in between, round it).

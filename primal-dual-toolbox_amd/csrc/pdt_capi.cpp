@@ -2624,6 +2624,13 @@ struct pdt_cnn {
 
   // out = net(x)
   void forward(const float* x, float* out, int n, int h, int wd) {
+    const int rows = cnn_net_rows(nl, n, h, wd);
+    const int64_t px = int64_t(n) * h * wd;
+    if (rows && (out + 6 * px <= x || x + 2 * px <= out)) {
+      cnn_net(stream, layers().data(), nl, x, out, n, h, wd, rows);
+      HIPC(hipGetLastError());
+      return;
+    }
     const void* in = hidden(x, n, h, wd);
     cnn_conv_last(stream, in, wk[nl - 1].p, b(nl - 1), out, n, h, wd);
     HIPC(hipGetLastError());

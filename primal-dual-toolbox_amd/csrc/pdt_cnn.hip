@@ -24,6 +24,7 @@
 #include <cstdint>
 
 #include "pdt_cnn.hpp"
+#include "pdt_pixel.hpp"
 
 namespace pdt {
 
@@ -32,6 +33,7 @@ namespace {
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 // two floats at 4-byte alignment (the caller's arrays)
 struct __attribute__((packed, aligned(4))) F2 {
@@ -42,6 +44,9 @@ constexpr int kConvThreads = 256;  // 4 waves, each on its own strips
 
 __device__ __forceinline__ f4 mfma(const bf8& a, const bf8& b, const f4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f16 mfma(const bf8& a, const bf8& b, const f16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
 // v where m is all ones, 0 where it is 0
@@ -344,6 +349,246 @@ __global__ __launch_bounds__(kConvThreads) void conv8_kernel(const __bf16* __res
         for (int t = 0; t < 2; ++t) acc[t] = mfma(wt[k][t], f[k], acc[t]);
       conv_store<2, EPI_MASK_BF16>(acc, b, (base + y) * w + x, x < w, out, ax, 0.f, ss);
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The whole network on a strip (inference): a workgroup has one wave per
+// layer, and rows of activations go from wave to wave through LDS.  At step t
+// wave l takes the row that wave l - 1 wrote at step t - 1 (32 pixels x 32
+// channels), adds it to the sums of the three output rows that it touches, and
+// writes the row it completes; the first wave gathers the input, the last one
+// stores the output.  One barrier a step.  The weights of a layer stay in its
+// wave's registers.  Of the 32 columns one on each side is lost per layer
+// after the first, of the rows as many above and below, and the pipeline takes
+// two steps a layer to fill.  Activations outside the image are zero, as the
+// layers' zero padding has them, and the products are added in the order of
+// the per-layer kernels: the outputs are the same bits.
+// Bound by a hidden wave's chain: 18 matrix instructions (576 clocks), the LDS
+// round trip, the rounding and the barrier, 0.45 us a step (0.60 us with
+// 16 x 16 tiles and taps gathered from memory).  Depth 5, a call: 1 x 320 x
+// 320 30 us (46 in five launches), 4 x 320 x 320 61 (84), 16 x 320 x 320 186
+// (255).
+// ---------------------------------------------------------------------------
+constexpr int kNetCols = 32;        // columns of a strip, halo included
+constexpr int kNetPix = kNetCols + 2;  // a staged row has one unused pixel on either side
+constexpr int kNetBlocks = 256;     // workgroups at a time: one per compute unit (registers)
+constexpr int kNetLayers = 8;       // deepest network (its halo leaves 18 columns)
+
+// LDS slot (8 channels each) of chunk c of staged pixel p: any 16 neighbouring
+// pixels' chunks c lie on different banks.
+__device__ __forceinline__ int net_slot(int p, int c) { return p * 4 + (c ^ ((p >> 2) & 3)); }
+
+// Steps of a workgroup that stores R rows, a multiple of three.
+__host__ __device__ constexpr int net_steps(int R, int depth) { return (R + 3 * (depth - 1) + 2) / 3 * 3; }
+
+// The first layer: its rows to `next`.  One load per input row (a pixel per
+// lane), six rows ahead, rounded to bf16 into a ring of three rows in LDS; a
+// lane gathers its taps 4 g .. 4 g + 3 (k = 2 tap + channel) from there, those
+// past the ninth from a cell that holds zero.
+__device__ __forceinline__ void net_first(const bf8* wk, const float* bias, const float* in, bf8* next, uint32_t* taps,
+                                          int steps, size_t base, int ya, int h, int xr, int w) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const bf8 w0 = wk[lane], w1 = wk[64 + lane];
+  float b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) b[i] = bias[g * 8 + i];
+  const int xl = xr - 1 + lane, xc = min(max(xl, 0), w - 1);
+  const bool in_cols = lane < kNetPix && xl >= 0 && xl < w;
+  if (lane == 0) taps[3 * kNetPix] = 0;
+  auto load = [&](F2& q, int yr) {
+    q = *reinterpret_cast<const F2*>(in + 2 * ((base + min(max(yr, 0), h - 1)) * w + xc));
+  };
+  auto stage = [&](F2 q, int yr, int slot) {
+    asm volatile("" : "+v"(q.a), "+v"(q.b));  // not rounded, hence not waited for, before its step
+    const bool ok = in_cols && yr >= 0 && yr < h;
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    const bf2 v = {__bf16(ok ? q.a : 0.f), __bf16(ok ? q.b : 0.f)};
+    if (lane < kNetPix) taps[slot * kNetPix + lane] = __builtin_bit_cast(uint32_t, v);
+  };
+  // cells of the taps for row slot (0, 1, 2) of the output row
+  int cell[3][4], step2[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int tap = 4 * g + j;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) cell[k][j] = tap < 9 ? (k + 2 + tap / 3) % 3 * kNetPix + c + tap % 3 : 3 * kNetPix;
+    step2[j] = tap < 9 ? 16 : 0;
+  }
+  // row ya + t in slot t % 3 (t counted from -1 as 2)
+  auto step = [&](int t, int k, F2& q) {
+    const int yr = ya + t;
+    stage(q, yr + 1, (k + 1) % 3);
+    load(q, yr + 7);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const int x = xr + m * 16 + c;
+      u4 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = taps[cell[k][j] + m * step2[j]];
+      const bf8 f = __builtin_bit_cast(bf8, v);
+      const f4 z = {0.f, 0.f, 0.f, 0.f};
+      const f4 acc[2] = {mfma(w0, f, z), mfma(w1, f, z)};
+      bf8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = __bf16(fmaxf(acc[i / 4][i % 4] + b[i], 0.f));
+      next[(t & 1) * (kNetPix * 4) + net_slot(m * 16 + c + 1, g)] =
+          keep(o, yr >= 0 && yr < h && x >= 0 && x < w ? ~0u : 0u);
+    }
+    wg_barrier();
+  };
+  F2 p, q, r[6];
+  load(p, ya - 1);
+  load(q, ya);
+#pragma unroll
+  for (int i = 0; i < 6; ++i) load(r[i], ya + 1 + i);
+  stage(p, ya - 1, 2);
+  stage(q, ya, 0);
+  for (int t = 0; t < steps; t += 3) {
+    step(t, 0, r[0]);
+    step(t + 1, 1, r[1]);
+    step(t + 2, 2, r[2]);
+    if ((t += 3) >= steps) break;
+    step(t, 0, r[3]);
+    step(t + 1, 1, r[4]);
+    step(t + 2, 2, r[5]);
+  }
+}
+
+// A hidden layer: its rows to `next`.  32 x 32 matrix tiles, channels by
+// pixels: half the instructions of 16 x 16 tiles, which one wave per SIMD does
+// not issue back to back (28 clocks each instead of 16; 32 clocks of 32 here).
+__device__ __forceinline__ void net_hidden(const bf8* wk, const float* bias, const bf8* prev, bf8* next, int l,
+                                           int steps, int ya, int h, int xr, int w) {
+  const int lane = threadIdx.x & 63, half = lane >> 5, c = lane & 31;
+  // Row c of the tile is the output channel that leaves a lane with channels
+  // 16 half .. 16 half + 15 of its pixel.
+  const int ch = 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
+  bf8 wt[9][2];
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      wt[k][s] = wk[(k * 2 + ((ch >> 2) & 1)) * 64 + (2 * s + half) * 16 + (ch >> 3) * 4 + (ch & 3)];
+  float b[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) b[i] = bias[16 * half + i];
+  f16 r0, r1, r2;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r0[i] = r1[i] = r2[i] = 0.f;
+  const int x = xr + c;
+  const bool in_cols = x >= 0 && x < w;
+  auto step = [&](int t, f16& first, f16& mid, f16& last) {
+    const bf8* in = prev + ((t - 1) & 1) * (kNetPix * 4);
+    bf8 f[3][2];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) f[d][s] = in[net_slot(c + d, 2 * s + half)];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) first[i] = 0.f;
+    // The row that is completed runs ahead, so that its bias, rounding and
+    // store are beside the products of the other two.
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      last = mfma(wt[6 + j / 2][j & 1], f[j / 2][j & 1], last);
+      const int k = j >> 1;
+      if (j & 1)
+        first = mfma(wt[k / 2][k & 1], f[k / 2][k & 1], first);
+      else
+        mid = mfma(wt[3 + k / 2][k & 1], f[k / 2][k & 1], mid);
+    }
+#pragma unroll
+    for (int k = 3; k < 6; ++k) {
+      mid = mfma(wt[3 + k / 2][k & 1], f[k / 2][k & 1], mid);
+      first = mfma(wt[k / 2][k & 1], f[k / 2][k & 1], first);
+    }
+    const int yo = ya + t - 2 * l;
+    const unsigned mask = yo >= 0 && yo < h && in_cols ? ~0u : 0u;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      bf8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = __bf16(fmaxf(last[8 * q + i] + b[8 * q + i], 0.f));
+      next[(t & 1) * (kNetPix * 4) + net_slot(c + 1, 2 * half + q)] = keep(o, mask);
+    }
+    wg_barrier();
+  };
+  for (int t = 0; t < steps; t += 3) {
+    step(t, r0, r1, r2);
+    step(t + 1, r2, r0, r1);
+    step(t + 2, r1, r2, r0);
+  }
+}
+
+// The last layer: rows [y0, y1) and columns [s0, s1) to y.
+__device__ __forceinline__ void net_last(const bf8* wk, const float* bias, const bf8* prev, float* y, int l, int steps,
+                                         size_t base, int ya, int y0, int y1, int xr, int s0, int s1, int w) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  bf8 wt[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) wt[k] = wk[k * 64 + lane];
+  float b[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = g * 4 + i < 6 ? bias[g * 4 + i] : 0.f;
+  f4 r0[2][1], r1[2][1], r2[2][1];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) r0[m][0] = r1[m][0] = r2[m][0] = f4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int t, f4 (&first)[2][1], f4 (&mid)[2][1], f4 (&last)[2][1]) {
+    const bf8* in = prev + ((t - 1) & 1) * (kNetPix * 4);
+    bf8 f[3][2];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) f[d][m] = in[net_slot(m * 16 + c + d, g)];
+    first[0][0] = first[1][0] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        last[m][0] = mfma(wt[6 + d], f[d][m], last[m][0]);
+        first[m][0] = mfma(wt[d], f[d][m], first[m][0]);
+        mid[m][0] = mfma(wt[3 + d], f[d][m], mid[m][0]);
+      }
+    const int yo = ya + t - 2 * l;
+    if (yo >= y0 && yo < y1)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const int x = xr + m * 16 + c;
+        double ss = 0;
+        conv_store<1, EPI_F32>(last[m], b, (base + yo) * w + x, x >= s0 && x < s1, y, Aux<EPI_F32>{}, 0.f, ss);
+      }
+    wg_barrier();
+  };
+  for (int t = 0; t < steps; t += 3) {
+    step(t, r0, r1, r2);
+    step(t + 1, r2, r0, r1);
+    step(t + 2, r1, r2, r0);
+  }
+}
+
+__global__ __launch_bounds__(64 * kNetLayers) __attribute__((amdgpu_waves_per_eu(2))) void net_kernel(
+    const float* __restrict__ in, float* y, CnnLayers ls, int depth, int n, int h, int w, int R) {
+  __shared__ __attribute__((aligned(16))) bf8 ring[(kNetLayers - 1) * 2 * kNetPix * 4];
+  __shared__ uint32_t taps[3 * kNetPix + 1];
+  const int halo = depth - 1, ow = kNetCols - 2 * halo, ns = (w + ow - 1) / ow, nc = (h + R - 1) / R;
+  const int id = xcd_block(blockIdx.x, gridDim.x), img = id / (ns * nc), r = id - img * ns * nc, cy = r / ns;
+  const int s0 = (r - cy * ns) * ow, s1 = min(w, s0 + ow), xr = s0 - halo;
+  const int y0 = cy * R, y1 = min(h, y0 + R), ya = y0 - halo;
+  const size_t base = size_t(img) * h;
+  const int steps = net_steps(R, depth);
+  const int l = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const CnnLayer& L = ls.l[l];
+  const bf8* wk = static_cast<const bf8*>(L.wk);
+  const float* bias = L.w + 9 * L.cin * L.cout;
+  const bf8* prev = ring + (l - 1) * 2 * (kNetPix * 4);
+  bf8* next = ring + l * 2 * (kNetPix * 4);
+  if (l == depth - 1) {
+    net_last(wk, bias, prev, y, l, steps, base, ya, y0, y1, xr, s0, s1, w);
+  } else if (l > 0) {
+    net_hidden(wk, bias, prev, next, l, steps, ya, h, xr, w);
+  } else {
+    net_first(wk, bias, in, next, taps, steps, base, ya, h, xr, w);
   }
 }
 
@@ -766,6 +1011,31 @@ void cnn_conv_last(hipStream_t st, const void* in, const void* wk, const float* 
   PDT_CONV(kWavesLast, (conv32_kernel<1, EPI_F32>), static_cast<const __bf16*>(in), static_cast<const bf8*>(wk), b, y, nullptr,
            nullptr);
 }
+int cnn_net_rows(int depth, int n, int h, int w) {
+  if (depth < 2 || depth > kNetLayers) return 0;
+  const int ow = kNetCols - 2 * (depth - 1);
+  const int64_t strips = int64_t(n) * ((w + ow - 1) / ow);
+  const double kpx = 1e-3 * n * h * w;
+  double best = 3.9 * depth + kpx * (0.031 + 0.034 * (depth - 2));
+  const double step = depth == 2 ? 0.28 : depth <= 5 ? 0.45 : depth == 6 ? 0.50 : 0.69;
+  int rows = 0;
+  for (int rounds = 1; rounds <= 32; ++rounds) {
+    const int64_t chunks = kNetBlocks * rounds / strips;
+    if (chunks == 0) continue;
+    const int R = int((h + chunks - 1) / chunks + 2) / 3 * 3;
+    const double t = rounds * (1.4 + step * net_steps(R, depth));
+    if (t < best) best = t, rows = R;
+  }
+  return rows;
+}
+void cnn_net(hipStream_t st, const CnnLayer* ls, int depth, const float* x, float* y, int n, int h, int w, int rows) {
+  const int ow = kNetCols - 2 * (depth - 1), ns = (w + ow - 1) / ow;
+  CnnLayers t{};
+  for (int l = 0; l < depth; ++l) t.l[l] = ls[l];
+  hipLaunchKernelGGL(net_kernel, dim3(n * ns * ((h + rows - 1) / rows)), dim3(64 * depth), 0, st, x, y, t, depth, n, h, w,
+                     rows);
+}
+
 void cnn_conv_last_mse(hipStream_t st, const void* in, const void* wk, const float* b, const float* t, void* dz,
                        double* part, int n, int h, int w) {
   PDT_CONV(kWavesLast, (conv32_kernel<1, EPI_MSE>), static_cast<const __bf16*>(in), static_cast<const bf8*>(wk), b, dz, t, part);

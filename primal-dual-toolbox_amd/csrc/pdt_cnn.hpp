@@ -38,6 +38,18 @@ void cnn_pack_weights(hipStream_t st, const CnnLayer* ls, int count);
 void cnn_conv_first(hipStream_t st, const float* x, const void* wk, const float* b, void* out, int n, int h, int w);
 void cnn_conv_hidden(hipStream_t st, const void* in, const void* wk, const float* b, void* out, int n, int h, int w);
 void cnn_conv_last(hipStream_t st, const void* in, const void* wk, const float* b, float* y, int n, int h, int w);
+// The whole network in one launch, workgroups of `rows` output rows by a strip
+// of columns; x and y must not overlap.  cnn_net_rows: the rows that make it
+// fastest, or 0 where the per-layer launches are faster.  Microseconds, fitted
+// to depths 2 .. 8 and 1 .. 16 images of 8 to 1000 pixels a side: 1.4 + 0.45
+// per row and pipeline step for each round of 256 workgroups (0.28 at depth 2,
+// 0.69 from depth 7, where two hidden layers share a SIMD), against 3.9 per
+// launch and 0.031 + 0.034 per hidden layer for every thousand pixels.  Depth
+// 5: 1 x 320 x 320 30 against 46 us, 16 x 320 x 320 186 against 255; 1024 x 8
+// x 8 (a third of each strip used, four rounds) 62 against 41; depth 2, 16 x
+// 320 x 320 118 against 72; depth 8, 16 x 320 x 320 516 against 420.
+int cnn_net_rows(int depth, int n, int h, int w);
+void cnn_net(hipStream_t st, const CnnLayer* ls, int depth, const float* x, float* y, int n, int h, int w, int rows);
 // The last layer of a training pass: y = conv(in) + b is not stored but
 // compared with t: the loss 1/(2m) sum (y - t)^2 over the m = 6 n h w outputs
 // as cnn_mse_blocks fp64 partial sums, and dz = (y - t) / m in bf16, padded to

@@ -206,4 +206,15 @@ __device__ __forceinline__ int xcd_item(int b, int n) {
   return x * q + min(x, r) + k;
 }
 
+// Workgroup barrier with its own wait for the wave's LDS accesses.  (At the
+// head of a loop whose last LDS store is at its end, the compiler drops the
+// wait of __syncthreads, which it finds satisfied on the way into the loop:
+// read in this build's assembly, where the barrier let a wave read the edge
+// row of the iteration before.)
+__device__ __forceinline__ void wg_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#endif
+}
+
 }  // namespace pdt

@@ -199,21 +199,15 @@ FftPlanD make_plan(int n, bool dbl) {
   return pl;
 }
 
-// Largest tiles that fit the LDS of a workgroup: coils per row work item and
-// columns per column group of the MRI passes.
+// Coils per row work item of the MRI passes that fit the LDS of a workgroup.
 int max_cb(int dt, int W, int nc, int C) {
   int cb = std::max(C, 1);
   while (cb > 1 && lds_rows_bytes(dt, cb, W, nc) > init_kernel_attrs()) --cb;
   return cb;
 }
-int max_cg(int dt, int Hk, int nc) {
-  int cg = std::max(nc, 1);
-  while (cg > 1 && lds_cols_bytes(dt, cg, Hk) > init_kernel_attrs()) --cg;
-  return cg;
-}
-// Default tiles before any autotuning: 4 coils per row item, 2 columns per
-// column group (temporally blocked denoising: block_choose).
-constexpr int kDefaultCb = 4, kDefaultCg = 2;
+// Default tiles before any autotuning: 4 coils per row item (columns per
+// column group: default_cg; temporally blocked denoising: block_choose).
+constexpr int kDefaultCb = 4;
 
 }  // namespace
 
@@ -413,7 +407,7 @@ struct pdt_op {
     if (lds_cols_bytes(dt, 1, Hk) > init_kernel_attrs() || lds_rows_bytes(dt, 1, W, ncols) > init_kernel_attrs())
       fail(PDT_ERR_UNSUPPORTED, prefix() + "transform length too large for the LDS passes");
     cb_out = std::min(kDefaultCb, max_cb(dt, W, ncols, C));
-    cg_out = std::min(kDefaultCg, max_cg(dt, Hk, ncols));
+    cg_out = std::min(default_cg(Hk), max_cg(dt, Hk, ncols));
     lr = lds_rows_bytes(dt, cb_out, W, ncols);
     lc = lds_cols_bytes(dt, cg_out, Hk);
   }
@@ -824,7 +818,7 @@ struct Engine {
   bool fp16 = false;
   bool pair_duals = true;  // TGV denoising: the dual step as 2-pixel vectors (even widths)
   int force_dpx = 0;       // dual step pixels per thread (0: cache / default)
-  int force_cb = 0, force_cg = 0, force_rpi = 0, force_cb_a = 0;  // autotuner overrides (0: cache / default; cb_a -1: default)
+  int force_cb = 0, force_cg = 0, force_rpi = 0, force_cb_a = 0;  // autotuner overrides (0: cache / default; cg, cb_a -1: default)
   int force_wpc[4] = {-1, -1, -1, -1};  // occupancy caps (-1: cache; 0: none)
   int force_tb[3] = {0, 0, -1};         // blocked ROF tiles (tb[2] -1: cache / default; 0: off)
   int force_unpaired = -1;              // MRI: 1 three launches per iteration, 0 pairs where possible (-1: cache)
@@ -897,12 +891,17 @@ struct Engine {
         maxC = std::max(maxC, s->op->C);
         maxNc = std::max(maxNc, s->op->ncols);
       }
+      int cg_max = maxNc, cg_def = maxNc;  // of every slice's column length
+      for (auto* s : sv) {
+        cg_max = std::min(cg_max, max_cg(dt, s->op->Hk, maxNc));
+        cg_def = std::min(cg_def, default_cg(s->op->Hk));
+      }
       key = mri_key(sv);
       TuneVal tv = tune_lookup(key);
       for (int i = 0; i < 4; ++i) L.wpc[i] = force_wpc[i] >= 0 ? force_wpc[i] : tv.wpc[i];
       unpaired = force_unpaired >= 0 ? force_unpaired != 0 : tv.unpaired != 0;
       cb = force_cb > 0 ? force_cb : tv.cb > 0 ? tv.cb : kDefaultCb;
-      cg = force_cg > 0 ? force_cg : tv.cg > 0 ? tv.cg : kDefaultCg;
+      cg = force_cg > 0 ? force_cg : force_cg < 0 ? cg_def : tv.cg > 0 ? tv.cg : cg_def;
       // default adjoint grouping: every coil of a row in one wide block where
       // a single slice's straight-line adjoint path fits (with the u and v
       // steps in that pass and, by default, paired iterations), else cb
@@ -912,7 +911,7 @@ struct Engine {
       cb_a = force_cb_a > 0 ? force_cb_a : force_cb_a < 0 ? def_cb_a : tv.cb_a > 0 ? tv.cb_a : def_cb_a;
       cb = std::max(1, std::min(cb, max_cb(dt, maxW, maxNc, maxC)));
       cb_a = std::max(1, std::min(cb_a, max_cb(dt, maxW, maxNc, maxC)));
-      cg = std::max(1, std::min(cg, max_cg(dt, maxHk, maxNc)));
+      cg = std::max(1, std::min(cg, cg_max));
       lr = lds_rows_bytes(dt, cb, maxW, maxNc);
       lra = lds_rows_bytes(dt, cb_a, maxW, maxNc);
       lc = lds_cols_bytes(dt, cg, maxHk);
@@ -2402,7 +2401,7 @@ int pdt_autotune(pdt_solver** solvers, int count, int reps, pdt_tiles* out, doub
       cbs.erase(std::unique(cbs.begin(), cbs.end()), cbs.end());
       for (int cb : cbs)
         if (cb <= maxC)
-          for (int cg : {1, 2, 4}) {
+          for (int cg : {1, 2, 3, 4}) {
             cand.push_back({{cb, cg, 0, cb}, {0, 0, 0}, 0});
             if (cb != maxC) cand.push_back({{cb, cg, 0, maxC}, {0, 0, 0}, 0});
             // every coil in the adjoint row blocks: also the three-launch iteration
@@ -2523,7 +2522,7 @@ int pdt_set_tiles(pdt_solver** solvers, int count, const pdt_tiles* t) {
     e.plan_only = true;
     // zero or negative: the default, not a cached choice
     e.force_cb = t->cb > 0 ? t->cb : kDefaultCb;
-    e.force_cg = t->cg > 0 ? t->cg : kDefaultCg;
+    e.force_cg = t->cg > 0 ? t->cg : -1;  // (-1: the engine's default)
     e.force_rpi = t->rpi > 0 ? t->rpi : 1;
     e.force_cb_a = t->cb_a > 0 ? t->cb_a : -1;  // (-1: the engine's default grouping)
     for (int i = 0; i < 4; ++i) e.force_wpc[i] = std::max(0, std::min(t->wpc[i], 6));

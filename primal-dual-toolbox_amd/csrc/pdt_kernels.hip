@@ -172,7 +172,7 @@ template <class R> struct Dft<R, 8> {
   }
 };
 
-// Radices 6 and 10: even/odd split into two DFTs of half length m,
+// Radices 6, 10 and 12.  6 and 10: even/odd split into two DFTs of half length m,
 // X[k] = E[k] + w^k O[k], X[k + m] = E[k] - w^k O[k], w = exp(s i pi / m).
 template <class R> struct Dft<R, 6> {
   static __device__ __forceinline__ void run(Cx<R>* x, R s) {
@@ -188,6 +188,34 @@ template <class R> struct Dft<R, 6> {
     x[4] = e[1] - t1;
     x[2] = e[2] + t2;
     x[5] = e[2] - t2;
+  }
+};
+template <class R> struct Dft<R, 12> {
+  // X[k + 4 m] = sum_j w3^(j m) w12^(j k) Y_j[k], Y_j the 4-point DFT of
+  // x[j], x[j + 3], x[j + 6], x[j + 9]
+  static __device__ __forceinline__ void run(Cx<R>* x, R s) {
+    const R h = R(0.86602540378443864676);  // cos(pi / 6)
+    Cx<R> y[3][4];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[j][i] = x[j + 3 * i];
+      Dft<R, 4>::run(y[j], s);
+    }
+    y[1][1] = y[1][1] * Cx<R>{h, s * R(0.5)};
+    y[1][2] = y[1][2] * Cx<R>{R(0.5), s * h};
+    y[1][3] = muli(y[1][3], s);
+    y[2][1] = y[2][1] * Cx<R>{R(0.5), s * h};
+    y[2][2] = y[2][2] * Cx<R>{R(-0.5), s * h};
+    y[2][3] = -y[2][3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      Cx<R> z[3] = {y[0][k], y[1][k], y[2][k]};
+      Dft<R, 3>::run(z, s);
+      x[k] = z[0];
+      x[k + 4] = z[1];
+      x[k + 8] = z[2];
+    }
   }
 };
 template <class R> struct Dft<R, 10> {
@@ -1086,12 +1114,36 @@ __device__ __forceinline__ void dual_workgroup(const SliceDev& d, int nd, double
   const R w0 = ball_weight(sched_alpha<R>(d, d.alpha0, d.alpha0_end, k));
   const R w1 = ball_weight(sched_alpha<R>(d, d.alpha1, d.alpha1_end, k));
   const float rW = 1.0f / float(W);
-  double t[kGapTerms] = {0};
-  for (int i = pa + threadIdx.x; i < pe; i += NT) {
-    const int y = qdiv(i, W, rW), x = i - y * W;
-    dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, w0, w1, t);
+  // GAP: the sums are formed as by 256 threads whatever NT is (wave w takes
+  // the pixels of waves w, w + NT / 64, ... of those), so that every launch
+  // that carries these workgroups finds the same bits.
+  constexpr int VT = GAP ? kBlock : NT, VW = VT / 64, NW = NT / 64;
+  __shared__ double red[GAP ? VW * kGapTerms : 1];
+  const int lane = threadIdx.x & 63;
+  for (int vw = threadIdx.x >> 6; vw < VW; vw += NW) {
+    double t[kGapTerms] = {0};
+    for (int i = pa + vw * 64 + lane; i < pe; i += VT) {
+      const int y = qdiv(i, W, rW), x = i - y * W;
+      dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, w0, w1, t);
+    }
+    if (GAP) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        double v = t[k];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+        if (lane == 0) red[vw * kGapTerms + k] = v;
+      }
+    }
   }
-  if (GAP) block_sum<3, NT>(reinterpret_cast<double(&)[3]>(t), part + size_t(b) * kGapTerms);
+  if (GAP) {
+    __syncthreads();
+    if (threadIdx.x < 3) {
+      double v = 0;
+      for (int w = 0; w < VW; ++w) v += red[w * kGapTerms + threadIdx.x];
+      part[size_t(b) * kGapTerms + threadIdx.x] = v;
+    }
+  }
 }
 
 template <class R, int MODE, bool GAP, int NT, int NF>
@@ -1348,6 +1400,188 @@ __global__ __launch_bounds__(NT) void k_cols(const SliceDev* sl, const int2* ite
   for (int e = threadIdx.x; e < ncg * H; e += NT) {
     const int yy = qdiv(e, ncg, rncg), cl = e - yy * ncg;
     T2[yy * nc + cl] = scale * res[lp<NF>(cl * Hk + fshift_src(yy + y0, Hk))];
+  }
+  if (GAP) block_sum<2, NT>(t, part + size_t(li) * kGapTerms);
+}
+
+// Column pass of the lengths 8 M 8 (with_direct_cols): a thread does one
+// butterfly of every stage, and what comes before the first stage, between the
+// two transforms and after the last one stays in its registers.  The first
+// stage reads T1; the last stage of the forward transform leaves outputs
+// i + q n / 8 in a thread, which are the inputs of the first stage of the
+// inverse transform, so the prox of those samples is done on registers; the
+// last stage writes T2.  Four barriers and four passes through LDS, where the
+// general kernel has eight and nine.
+// Bound by this chain (descriptor, loads, six stages, stores) with every
+// workgroup resident at once, not by its bytes.  Per launch, general kernel
+// before, this one after: 640 points, 15 coils x 80 columns with the dual step
+// 11.9 -> 10.3 us; 768 points, 15 x 117 16.3 -> 13.4; 512 points in double
+// precision (a runtime plan before), 8 x 64 12.9 -> 8.3.
+// At most CS columns per group (max_cg): two of 640 points (160 threads) were
+// faster than three or four, 27.8 against 28.4 and 29.0 us per iteration, and
+// two of 512 in double than four.
+template <class R, int NF>
+struct ColShape {
+  static constexpr int M = NF / 64, NR = NF / 8;  // middle radix; butterflies of a radix-8 stage
+  static constexpr int CS = NR > 80 ? 2 : 160 / NR;  // columns at most
+  static constexpr int NT = (CS * (NR > 64 ? NR : 64) + 63) / 64 * 64;
+  static constexpr int NP = NF + NF / 8;          // LDS slots of a column, one pad slot per 8 elements
+  static constexpr size_t lds = (NF + 2 * size_t(CS) * NP) * sizeof(Cx<R>);
+};
+template <class R, int CMODE, bool GAP, int NF, int DUAL = 0>
+__global__ __launch_bounds__((ColShape<R, NF>::NT)) void k_cols_direct(const SliceDev* sl, const int2* items, int nitems,
+                                                                     int cg, double* part, int ndual,
+                                                                     double* part_dual) {
+  using C = Cx<R>;
+  using Sh = ColShape<R, NF>;
+  constexpr int CS = Sh::CS, M = Sh::M, NR = Sh::NR, NT = Sh::NT, NP = Sh::NP, NRP = NR + NR / 8, Hk = NF;
+  static_assert(NF == 64 * M && NR % 8 == 0, "8 M 8, padded");
+  extern __shared__ char smem_raw[];
+  if (DUAL != 0 && int(blockIdx.x) >= nitems) {
+    const SliceDev& d = sl[0];
+    if (!slice_active(d)) return;
+    dual_workgroup<R, DUAL, GAP, NT>(d, ndual, part_dual);
+    return;
+  }
+  const int li = xcd_item(blockIdx.x, nitems);
+  const int2 it = items ? items[li] : make_int2(0, li);  // null: the dense single-slice list
+  const SliceDev& d = sl[it.x];
+  const int W = d.W, H = d.H, y0 = d.y0, nc = d.ncols;
+  const int c = it.y / d.ngroups, g = it.y - c * d.ngroups;
+  const R scale = R(1) / sqrt(R(W) * R(Hk));
+  const R sigma = R(d.sigma), lambda = R(d.lambda), inv_sl = rcp(R(1) + sigma * lambda);
+  C* const tw = reinterpret_cast<C*>(smem_raw);
+  C* const bufA = tw + Hk;
+  C* const bufB = bufA + CS * NP;
+  const auto T1 = gptr<const C>(d.T1) + size_t(c) * H * nc;
+  const auto T2 = gptr<C>(d.T2) + size_t(c) * H * nc;
+  const auto fk = gptr<const C>(d.fk) + size_t(c) * nc * Hk;
+  const auto rk = gptr<C>(d.rk) + size_t(c) * nc * Hk;
+  const auto Mc = gptr<const R>(d.Mc);
+  const auto cols = gptr<const int>(d.cols);
+  const auto in = gptr<const C>(d.op_in) + size_t(c) * Hk * W;
+  const auto out = gptr<C>(d.op_out) + size_t(c) * Hk * W;
+  // A thread's butterflies: the stages at T1 and T2 take columns fastest (the
+  // columns of a row are contiguous there), the stages at the prox the i of a
+  // column (f, r and the mask are contiguous along it), the middle stages one
+  // column per wave.
+  const int ca = threadIdx.x % CS, ia = threadIdx.x / CS;
+  const int cp = threadIdx.x / NR, ip = threadIdx.x - cp * NR;
+  const int cm = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), im = threadIdx.x & 63;
+  double t[2] = {0, 0};
+  Staged<C, NF, NT> s_tw;
+  s_tw.load(gptr<const C>(d.planH.tw), Hk);
+  // sample kfe of the transform's element i + q n / 8 (fftshift of an even length)
+  auto kfe = [](int i, int q) { return i + NR * ((q + 4) & 7); };
+  // radix-M stage of the middle: bufA -> bufB
+  auto middle = [&](bool act, bool inv) {
+    if (act) {
+      const int kk = im & 7;
+      const C* a = bufA + cm * NP + im + im / 8;
+      C z[M];
+      z[0] = a[0];
+#pragma unroll
+      for (int j = 1; j < M; ++j) z[j] = a[72 * j] * twd(tw, 8 * j * kk, inv);
+      Dft<R, M>::run(z, inv ? R(1) : R(-1));
+      C* b = bufB + cm * NP + (im / 8) * (9 * M) + kk;
+#pragma unroll
+      for (int q = 0; q < M; ++q) b[9 * q] = z[q];
+    }
+    __syncthreads();
+  };
+  const int ks0 = g * cg, ncs = min(cg, nc - ks0);
+  const bool acta = ia < NR && ca < ncs, actp = cp < ncs, actm = cm < ncs;
+  const int kp = ks0 + (actp ? cp : 0), e0 = kp * Hk + (actp ? ip : 0);
+  C x[8], pf[8], pr[8];
+  R pm[8];
+  bool ok[8];
+  // branch-free loads, so that the compiler's wait for the first ones counts
+  // those after them (lanes without work and zero-padded rows load one valid
+  // element, unused)
+  if (CMODE != CM_ADJ) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int yy = kfe(ia, j) - y0;
+      ok[j] = acta && yy >= 0 && yy < H;
+      x[j] = T1[ok[j] ? yy * nc + ks0 + ca : 0];
+    }
+  }
+  const int col = CMODE == CM_SOLVE ? 0 : int(cols[kp]);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int e = e0 + kfe(0, q);
+    pm[q] = Mc[e];
+    if (CMODE == CM_SOLVE) {
+      pf[q] = fk[e];
+      pr[q] = rk[e];
+    } else if (CMODE == CM_ADJ) {
+      pf[q] = in[size_t((actp ? ip : 0) + kfe(0, q)) * W + col];
+    }
+  }
+  if (!slice_active(d)) return;  // after the loads are issued, before any store
+  s_tw.store(tw, Hk);
+  if (CMODE != CM_ADJ) {
+    // forward: 8, M, 8
+    if (acta) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = csel(ok[j], x[j], pzero<C>());
+      Dft<R, 8>::run(x, R(-1));
+#pragma unroll
+      for (int q = 0; q < 8; ++q) bufA[ca * NP + 9 * ia + q] = x[q];
+    }
+    __syncthreads();
+    middle(actm, false);
+    if (actp) {
+      const C* b = bufB + cp * NP + ip + ip / 8;
+      x[0] = b[0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) x[j] = b[j * NRP] * twd(tw, j * ip, false);
+      Dft<R, 8>::run(x, R(-1));
+    }
+  }
+  if (actp) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (CMODE == CM_ADJ) {
+        x[q] = pm[q] * pf[q];
+        continue;
+      }
+      const C a = (pm[q] * scale) * x[q];
+      if (CMODE == CM_FWD) {
+        out[size_t(kfe(ip, q)) * W + col] = a;
+        continue;
+      }
+      // prox of r on A ubar - f: TGV_prox_r_kernel (tgv_kernels.cuh:212-223)
+      const C tmp = a - pf[q];
+      const C rn = (pr[q] + sigma * tmp) * inv_sl;
+      rk[e0 + kfe(0, q)] = rn;
+      if (GAP) {
+        t[0] += dabs2(tmp);
+        t[1] += dabs2(tmp - lambda * rn);
+      }
+      x[q] = pm[q] * rn;
+    }
+    if (CMODE != CM_FWD) {
+      // inverse: 8, M, 8
+      Dft<R, 8>::run(x, R(1));
+#pragma unroll
+      for (int q = 0; q < 8; ++q) bufA[cp * NP + 9 * ip + q] = x[q];
+    }
+  }
+  if (CMODE == CM_FWD) return;
+  __syncthreads();
+  middle(actm, true);
+  if (acta) {
+    const C* b = bufB + ca * NP + ia + ia / 8;
+    x[0] = b[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) x[j] = b[j * NRP] * twd(tw, j * ia, true);
+    Dft<R, 8>::run(x, R(1));
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int yy = kfe(ia, q) - y0;
+      if (yy >= 0 && yy < H) T2[yy * nc + ks0 + ca] = scale * x[q];
+    }
   }
   if (GAP) block_sum<2, NT>(t, part + size_t(li) * kGapTerms);
 }
@@ -2148,6 +2382,31 @@ static void with_fft_len(int n, Fn&& fn) {
   fn(std::integral_constant<int, 0>{});
 }
 
+// with_fft_len for the column lengths without k_cols_direct (N = 0: the
+// runtime plan, for any length).
+template <class R, class Fn>
+static void with_other_len(int n, Fn&& fn) {
+  if constexpr (std::is_same<R, float>::value) {
+    if (n == 368) return fn(std::integral_constant<int, 368>{});
+    if (n == 736) return fn(std::integral_constant<int, 736>{});
+  }
+  fn(std::integral_constant<int, 0>{});
+}
+
+// Calls fn(std::integral_constant<int, N>) when columns of n have k_cols_direct.
+template <class Fn>
+static bool with_direct_cols(int n, Fn&& fn) {
+  switch (n) {
+    case 256: fn(std::integral_constant<int, 256>{}); return true;
+    case 320: fn(std::integral_constant<int, 320>{}); return true;
+    case 384: fn(std::integral_constant<int, 384>{}); return true;
+    case 512: fn(std::integral_constant<int, 512>{}); return true;
+    case 640: fn(std::integral_constant<int, 640>{}); return true;
+    case 768: fn(std::integral_constant<int, 768>{}); return true;
+    default: return false;
+  }
+}
+
 bool fft_len_compiled(int dtype, int n) {
   if (dtype != DT_C64 && dtype != DT_F32) return false;
   for (int m : kFftLengths)
@@ -2187,11 +2446,63 @@ static void launch_rows_adj(const Launch& L, bool gap) {
   }
 }
 
+int max_cg(int dtype, int Hk, int nc) {
+  int cg = nc > 1 ? nc : 1;
+  with_direct_cols(Hk, [&](auto nf) {
+    constexpr int CS = ColShape<float, decltype(nf)::value>::CS;
+    cg = cg < CS ? cg : CS;
+  });
+  while (cg > 1 && lds_cols_bytes(dtype, cg, Hk) > init_kernel_attrs()) --cg;
+  return cg;
+}
+int default_cg(int Hk) {
+  int cg = 2;
+  with_direct_cols(Hk, [&](auto nf) { cg = ColShape<float, decltype(nf)::value>::CS; });
+  return cg;
+}
+
+// Column pass (DUAL: with the dual step's workgroups, gap terms to pd).
+template <class R, int CMODE, bool GAP, int DUAL>
+static void launch_cols_gap(const Launch& L, const int2* items, int ndual, double* pd) {
+  constexpr int NC = kColThreads;
+  const size_t limit = init_kernel_attrs();
+  bool done = false;
+  with_direct_cols(L.fft_h, [&](auto nf) {
+    constexpr int NF = decltype(nf)::value;
+    using Sh = ColShape<R, NF>;
+    if (Sh::lds > limit) return;  // (a runtime that refuses more than 64 KB)
+    done = true;
+    PDT_LAUNCH_NT((k_cols_direct<R, CMODE, GAP, NF, DUAL>), L.ncolitems + ndual, Sh::NT, lds_occupancy(Sh::lds, L.wpc[WPC_COLS], limit), L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], ndual, pd);
+  });
+  if (done) return;
+  const size_t lds = lds_occupancy(L.lds_cols, L.wpc[WPC_COLS], limit);
+  with_other_len<R>(L.fft_h, [&](auto nf) {
+    constexpr int NF = decltype(nf)::value;
+    if constexpr (NF > 0 && CMODE == CM_SOLVE) {
+      if (L.cg <= kColPrefetchCols) {
+        PDT_LAUNCH_NT((k_cols<R, CMODE, GAP, NC, NF, true, DUAL>), L.ncolitems + ndual, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], ndual, pd);
+        return;
+      }
+    }
+    PDT_LAUNCH_NT((k_cols<R, CMODE, GAP, NC, NF, false, DUAL>), L.ncolitems + ndual, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], ndual, pd);
+  });
+}
+template <class R, int CMODE>
+static void launch_cols(const Launch& L, bool gap, const int2* items) {
+  if constexpr (CMODE == CM_SOLVE) {
+    if (gap) {
+      launch_cols_gap<R, CMODE, true, 0>(L, items, 0, nullptr);
+      return;
+    }
+  }
+  launch_cols_gap<R, CMODE, false, 0>(L, items, 0, nullptr);
+}
+
 // MRI stages: 0 rows_fwd, 1 cols, 2 rows_adj, 3 primal.  The FFT kernels are
 // picked by L.fft_w (row length) and L.fft_h (column length).
 template <class R, int MODE>
 static void mri_stage_m(const Launch& L, bool gap, int stage) {
-  constexpr int NR = kRowThreads, NC = kColThreads;
+  constexpr int NR = kRowThreads;
   if (stage == 0) {
     const size_t lds = lds_occupancy(L.lds_rows, L.wpc[WPC_FWD], init_kernel_attrs());
     with_fft_len<R>(L.fft_w, [&](auto nf) {
@@ -2202,20 +2513,7 @@ static void mri_stage_m(const Launch& L, bool gap, int stage) {
     });
   } else if (stage == 1) {
     if (L.ncolitems == 0) return;
-    const size_t lds = lds_occupancy(L.lds_cols, L.wpc[WPC_COLS], init_kernel_attrs());
-    with_fft_len<R>(L.fft_h, [&](auto nf) {
-      constexpr int NF = decltype(nf)::value;
-      const int2* items = L.dense ? nullptr : L.cols;
-      if constexpr (NF > 0) {
-        if (L.cg <= kColPrefetchCols) {
-          if (gap) PDT_LAUNCH_NT((k_cols<R, CM_SOLVE, true, NC, NF, true>), L.ncolitems, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], 0, nullptr);
-          else PDT_LAUNCH_NT((k_cols<R, CM_SOLVE, false, NC, NF, true>), L.ncolitems, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], 0, nullptr);
-          return;
-        }
-      }
-      if (gap) PDT_LAUNCH_NT((k_cols<R, CM_SOLVE, true, NC, NF>), L.ncolitems, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], 0, nullptr);
-      else PDT_LAUNCH_NT((k_cols<R, CM_SOLVE, false, NC, NF>), L.ncolitems, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], 0, nullptr);
-    });
+    launch_cols<R, CM_SOLVE>(L, gap, L.dense ? nullptr : L.cols);
   } else if (stage == 2) {
     with_fft_len<R>(L.fft_w, [&](auto nf) {
       constexpr int NF = decltype(nf)::value;
@@ -2242,20 +2540,9 @@ static void mri_stage(const Launch& L, int kind, bool gap, int stage) {
 // items' and the row items' as in those passes.
 template <class R, int MODE, bool GAP>
 static void mri_pair_m(const Launch& L, int which) {
-  constexpr int NC = kColThreads, NW = kRowAdjThreadsWide;
+  constexpr int NW = kRowAdjThreadsWide;
   if (which == 0) {
-    const size_t lds = lds_occupancy(L.lds_cols, L.wpc[WPC_COLS], init_kernel_attrs());
-    double* const pd = L.part[0] + size_t(L.nrg) * kGapTerms;
-    with_fft_len<R>(L.fft_h, [&](auto nf) {
-      constexpr int NF = decltype(nf)::value;
-      if constexpr (NF > 0) {
-        if (L.cg <= kColPrefetchCols) {
-          PDT_LAUNCH_NT((k_cols<R, CM_SOLVE, GAP, NC, NF, true, MODE>), L.ncolitems + L.ndual, NC, lds, L.stream, L.sl, nullptr, L.ncolitems, L.cg, L.part[1], L.ndual, pd);
-          return;
-        }
-      }
-      PDT_LAUNCH_NT((k_cols<R, CM_SOLVE, GAP, NC, NF, false, MODE>), L.ncolitems + L.ndual, NC, lds, L.stream, L.sl, nullptr, L.ncolitems, L.cg, L.part[1], L.ndual, pd);
-    });
+    launch_cols_gap<R, CM_SOLVE, GAP, MODE>(L, nullptr, L.ndual, L.part[0] + size_t(L.nrg) * kGapTerms);
   } else {
     const size_t lds = lds_occupancy(L.lds_rows_a, L.wpc[WPC_ADJ], init_kernel_attrs());
     with_fft_len<R>(L.fft_w, [&](auto nf) {
@@ -2312,24 +2599,17 @@ void run_gap_reduce(const Launch& L, int kind, int dtype) {
 
 template <class R>
 static void op_forward(const Launch& L) {
-  constexpr int NR = kRowThreads, NC = kColThreads;
+  constexpr int NR = kRowThreads;
   with_fft_len<R>(L.fft_w, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     PDT_LAUNCH_NT((k_rows_fwd<R, M_OP, false, NR, NF>), L.nrg, NR, L.lds_rows, L.stream, L.sl, L.rowgroups, L.nrg, L.cb, L.part[0], 0);
   });
-  with_fft_len<R>(L.fft_h, [&](auto nf) {
-    constexpr int NF = decltype(nf)::value;
-    PDT_LAUNCH_NT((k_cols<R, CM_FWD, false, NC, NF>), L.ncolitems, NC, L.lds_cols, L.stream, L.sl, L.cols, L.ncolitems, L.cg, L.part[1], 0, nullptr);
-  });
+  launch_cols<R, CM_FWD>(L, false, L.cols);
 }
 
 template <class R>
 static void op_adjoint(const Launch& L) {
-  constexpr int NC = kColThreads;
-  with_fft_len<R>(L.fft_h, [&](auto nf) {
-    constexpr int NF = decltype(nf)::value;
-    PDT_LAUNCH_NT((k_cols<R, CM_ADJ, false, NC, NF>), L.ncolitems, NC, L.lds_cols, L.stream, L.sl, L.cols, L.ncolitems, L.cg, L.part[1], 0, nullptr);
-  });
+  launch_cols<R, CM_ADJ>(L, false, L.cols);
   with_fft_len<R>(L.fft_w, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     launch_rows_adj<R, M_OP, NF>(L, false);
@@ -2375,8 +2655,13 @@ static bool set_lds_attrs(int b) {
         set((const void*)&k_rows_adj<R, M_TGV, true, kRowAdjThreadsWide, NF, true, true>);
       }
     }
+  };
+  auto col = [&](auto nf) {
+    constexpr int NF = decltype(nf)::value;
     set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF>);
     set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF>);
+    set((const void*)&k_cols<R, CM_FWD, false, NC, NF>);
+    set((const void*)&k_cols<R, CM_ADJ, false, NC, NF>);
     if constexpr (std::is_same<R, float>::value) {
       set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, false, M_TV>);
       set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, false, M_TGV>);
@@ -2386,16 +2671,29 @@ static bool set_lds_attrs(int b) {
     if constexpr (NF > 0) {
       set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, true>);
       set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF, true>);
-      if constexpr (std::is_same<R, float>::value) {
-        set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, true, M_TV>);
-        set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, true, M_TGV>);
-        set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF, true, M_TV>);
-        set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF, true, M_TGV>);
-      }
+      set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, true, M_TV>);
+      set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, true, M_TGV>);
+      set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF, true, M_TV>);
+      set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF, true, M_TGV>);
     }
-    set((const void*)&k_cols<R, CM_FWD, false, NC, NF>);
-    set((const void*)&k_cols<R, CM_ADJ, false, NC, NF>);
   };
+  auto direct = [&](auto nf) {
+    constexpr int NF = decltype(nf)::value;
+    set((const void*)&k_cols_direct<R, CM_SOLVE, false, NF>);
+    set((const void*)&k_cols_direct<R, CM_SOLVE, true, NF>);
+    set((const void*)&k_cols_direct<R, CM_FWD, false, NF>);
+    set((const void*)&k_cols_direct<R, CM_ADJ, false, NF>);
+    if constexpr (std::is_same<R, float>::value) {
+      set((const void*)&k_cols_direct<R, CM_SOLVE, false, NF, M_TV>);
+      set((const void*)&k_cols_direct<R, CM_SOLVE, false, NF, M_TGV>);
+      set((const void*)&k_cols_direct<R, CM_SOLVE, true, NF, M_TV>);
+      set((const void*)&k_cols_direct<R, CM_SOLVE, true, NF, M_TGV>);
+    }
+  };
+  for (int n : kFftLengths) {
+    with_direct_cols(n, direct);
+    with_other_len<R>(n, col);  // (0 for the lengths of the line above)
+  }
   with_fft_len<R>(0, one);
   for (int n : kFftLengths)
     if (std::is_same<R, float>::value) with_fft_len<R>(n, one);

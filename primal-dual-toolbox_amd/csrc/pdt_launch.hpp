@@ -161,5 +161,9 @@ size_t init_kernel_attrs();
 // row pass uses them unpadded)
 size_t lds_rows_bytes(int dtype, int cb, int W, int nc, bool padded = true);
 size_t lds_cols_bytes(int dtype, int cg, int Hk);
+// Columns per column group: the most a launch takes, and the number without a
+// tuned or forced choice.
+int max_cg(int dtype, int Hk, int nc);
+int default_cg(int Hk);
 
 }  // namespace pdt

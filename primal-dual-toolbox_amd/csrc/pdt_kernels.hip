@@ -1616,10 +1616,37 @@ __device__ __forceinline__ void mri_primal_pixel(const SliceDev& d, int x, int y
 // must stay within 64 VGPRs (two blocks per CU), so it holds fewer.
 template <int NT> constexpr int rows_adj_ps() { return NT >= 1024 ? 6 : kPrefetch; }
 template <int NT> constexpr int rows_adj_pt() { return NT >= 1024 ? 2 : 4; }
-// the straight-line path loads its sensitivity slots unconditionally, so it
-// holds exactly as many as it may use (5 coils per thread group: 15 coils
-// on rows of 320, 20 on rows of 256)
-constexpr int kRowsAdjFusedSlots = 5;
+// The straight-line path loads its sensitivity slots unconditionally, so it
+// is built for as many as it uses: 5 coils for each thread group (15 coils on
+// rows of 320, 20 on rows of 256, 10 on rows of 384 and 512), and for the
+// padded lengths of two groups also 8 (16 coils).  8 slots spill a few
+// registers: 10 coils on rows of 384 take 30.5 us per iteration with them, 28
+// with 5; 12 coils 34 us, against 40 in three passes and k_mri_primal.
+constexpr int kFusedSlots = 5, kFusedSlotsMore = 8;
+constexpr bool fused_more_ok(int W) { return ct_pad_ok(W) && kRowAdjThreadsWide / W == 2; }
+// Coils per thread group.
+constexpr int fused_coils(int W, int C) {
+  const int ngs = kRowAdjThreadsWide / W < C ? kRowAdjThreadsWide / W : C;
+  return (C + ngs - 1) / ngs;
+}
+// Its LDS: twiddles, the coils' padded slots and the group sums (ct_pad_ok), or
+// two unpadded buffers.  (15 coils on rows of 384: 61 KB, two workgroups per
+// CU; with the 95 KB of two buffers one, and 28.7 us instead of 22.5.)
+constexpr size_t fused_lds(int W, int C, size_t esize) {
+  const int ngs = kRowAdjThreadsWide / W < C ? kRowAdjThreadsWide / W : C;
+  return (ct_pad_ok(W) ? size_t(W) + size_t(C) * (W + W / 8) + size_t(ngs) * W : size_t(W) * (1 + 2 * size_t(C))) * esize;
+}
+
+// Element e of a wave-uniform base: a 32-bit byte offset, so that the access
+// takes the base from scalar registers (fewer address instructions and
+// registers).  The offset must stay below 4 GB.
+template <class P>
+__device__ __forceinline__ auto& at(P base, uint32_t e) {
+  using T = std::remove_reference_t<decltype(*base)>;
+  using Byte = std::conditional_t<std::is_const<T>::value, const char, char>;
+  const auto b = (__attribute__((address_space(1))) Byte*)base;
+  return *(P)(b + e * uint32_t(sizeof(T)));
+}
 
 // The adjoint row pass of one row y holding all coils (FUSED in k_rows_adj):
 // T2 row -> ifftshift -> inverse PE-FFT -> fftshift -> * conj(S_c), summed
@@ -1628,10 +1655,10 @@ constexpr int kRowsAdjFusedSlots = 5;
 // (TGV_primal_u_noprox_kernel, tgv_kernels.cuh:432-467).  Load order: the
 // twiddles, the T2 gather, u and p of the primal step (their arithmetic
 // waits for them), then the sensitivities, which the FFT does not need.
-template <class R, int MODE, bool GAP, int NT, int NF, bool NEXT>
+template <class R, int MODE, bool GAP, int NT, int NF, int PS, bool NEXT>
 __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double* part_rows, char* smem_raw) {
   using C = Cx<R>;
-  constexpr int W = NF, PS = kRowsAdjFusedSlots, PT = rows_adj_pt<NT>();
+  constexpr int W = NF, PT = rows_adj_pt<NT>();
   // Lengths with the padded layout: one padded slot range per coil, whose
   // T2 scatter, transforms (fft_wave) and T1 entries one wavefront does
   // alone (coils wave, wave + NW, ...; lb holds the coil-group sums), so the
@@ -1639,7 +1666,7 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
   // workgroup-wide stages (lp without padding is the identity for them).
   constexpr bool IP = ct_pad_ok(NF);
   constexpr int NW = NT / 64, NPW = W + W / 8;  // waves; padded slots per coil
-  constexpr int SPW = (kRowsAdjFusedSlots * (NT / NF) + NW - 1) / NW;  // coils per wave
+  constexpr int SPW = (PS * (NT / NF) + NW - 1) / NW;  // coils per wave
   const int H = d.H, nc = d.ncols, ncb = d.C;
   const int ngs = min(NT / W, ncb), ch = (ncb + ngs - 1) / ngs;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
@@ -1661,11 +1688,12 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
   int pK[PT];
   if constexpr (IP) {
 #pragma unroll
-    for (int k = 0; k < PT; ++k) pK[k] = gcols[min(lane + 64 * k, nc - 1)];
+    for (int k = 0; k < PT; ++k) pK[k] = at(gcols, uint32_t(min(lane + 64 * k, nc - 1)));
 #pragma unroll
     for (int sq = 0; sq < SPW; ++sq)
 #pragma unroll
-      for (int k = 0; k < PT; ++k) pT[sq][k] = T2[min(wave + NW * sq, ncb - 1) * cstride + min(lane + 64 * k, nc - 1)];
+      for (int k = 0; k < PT; ++k)
+        pT[sq][k] = at(T2 + min(wave + NW * sq, ncb - 1) * cstride, uint32_t(min(lane + 64 * k, nc - 1)));
   } else {
 #pragma unroll
     for (int k = 0; k < PT; ++k) {
@@ -1687,23 +1715,23 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
   const int x = threadIdx.x;
   const bool upix = NEXT ? gi < ngs : x < W;
   const int xr = NEXT ? (gi < ngs ? gx : 0) : (x < W ? x : 0);
-  const size_t n = size_t(W) * H, i = size_t(y) * W + xr;
-  const auto pp = gptr<const C>(d.p);
-  const C e_uo = gptr<const C>(d.u)[i];
-  const C cx = pp[i], mx = pp[xr > 0 ? i - 1 : i];
-  const C cy = pp[n + i], my = pp[n + (y > 0 ? i - W : i)];
+  const size_t n = size_t(W) * H, row = size_t(y) * W;
+  const auto pp = gptr<const C>(d.p) + row;
+  const C e_uo = at(gptr<const C>(d.u) + row, uint32_t(xr));
+  const C cx = at(pp, uint32_t(xr)), mx = at(pp, uint32_t(max(xr - 1, 0)));
+  const C cy = at(pp + n, uint32_t(xr)), my = at(pp + n - (y > 0 ? W : 0), uint32_t(xr));
   // sensitivities, branch-free (spare slots load a valid element, unused)
   const int G = W * d.Hk;
-  const auto Sg = gptr<const C>(d.S) + size_t(y + d.y0) * W + gx;
+  const auto Sg = gptr<const C>(d.S) + size_t(y + d.y0) * W;
   C pS[PS];
 #pragma unroll
-  for (int k = 0; k < PS; ++k) pS[k] = Sg[size_t(min(gi * ch + k, ncb - 1)) * G];
+  for (int k = 0; k < PS; ++k) pS[k] = at(Sg, uint32_t(min(gi * ch + k, ncb - 1)) * uint32_t(G) + uint32_t(gx));
   if (!slice_active(d)) return;  // after the loads are issued, before any store
   // descriptor fields of the stores, read before the asm below (after it
   // the compiler no longer takes the descriptor for unmodified, and would
   // read them with vector loads at the end of the block)
-  const auto gu = gptr<C>(d.u);
-  const auto gub = gptr<C>(d.ub);
+  const auto gu = gptr<C>(d.u) + row;
+  const auto gub = gptr<C>(d.ub) + row;
   const auto gctl = gptr<int>(d.ctl);
   const int row_beg = d.row_beg;
   // div p = dmx + dmy (the same operations as dmx / dmy), formed here: the
@@ -1775,8 +1803,8 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
     const C un = e_uo + tau * (e_div - w);
     const C ubn = (R(1) + theta) * un - theta * e_uo;
     if (!NEXT || gi == 0) {  // (NEXT: one thread group stores and counts the pixel)
-      gu[i] = un;
-      gub[i] = ubn;
+      at(gu, uint32_t(xr)) = un;
+      at(gub, uint32_t(xr)) = ubn;
       if (GAP) t[0] += dabs2(w - e_div);
     }
     if constexpr (NEXT) {
@@ -1811,7 +1839,7 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
 #pragma unroll
           for (int k = 0; k < PT; ++k) {
             const int ks = lane + 64 * k, j = fshift_src(pK[k], W);
-            if (ks < nc) T1[size_t(cl) * H * nc + ks] = sp[j + (j >> 3)];
+            if (ks < nc) at(T1 + cl * cstride, uint32_t(ks)) = sp[j + (j >> 3)];
           }
         }
       }
@@ -1837,7 +1865,8 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
 // row y itself (MODE M_OP: writes A^* r to op_out).  The 1024-thread
 // variant on swz-permuted buffers is held to 64 VGPRs (its slot arithmetic
 // would take more), so that two workgroups share a CU.
-// FUSED (host-checked, see rows_adj_fused_ok): a compile-time row length, one
+// FUSED (sensitivity slots per thread; host-checked, see rows_adj_fused_ok): a
+// compile-time row length, one
 // coil group per row holding every coil (the u step follows in the block),
 // 2 W <= NT, the coil products in registers (every thread group's coils fit
 // its slots), the T2 row in registers, sensitivities present, and no v step
@@ -1849,13 +1878,13 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
 // from their new ubar row, which k_rows_fwd's row items would otherwise do
 // (rows_adj_fused).  Its gap-evaluation variant (one iteration in
 // gap_every) is not held to 64 VGPRs: within them it spilled.
-template <class R, int MODE, bool GAP, int NT, int NF, bool FUSED = false, bool NEXT = false>
+template <class R, int MODE, bool GAP, int NT, int NF, int FUSED = 0, bool NEXT = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 && NF > 0 && ct_pad_ok(NF) && !(GAP && NEXT) ? 8 : 1))) void k_rows_adj(const SliceDev* sl, const int2* items, int nitems, int cb,
                                                  double* part_rows, int nvstep) {
   extern __shared__ char smem_raw[];
   using C = Cx<R>;
-  static_assert(!FUSED || (NF > 0 && MODE != M_OP && NT == kRowAdjThreadsWide), "fused adjoint row path");
-  static_assert(!NEXT || FUSED, "next forward rows: the fused path");
+  static_assert(FUSED == 0 || (NF > 0 && MODE != M_OP && NT == kRowAdjThreadsWide), "fused adjoint row path");
+  static_assert(!NEXT || FUSED != 0, "next forward rows: the fused path");
   if (int(blockIdx.x) >= nitems) {
     // nvstep workgroups after the row items (a single slice): the v step of
     // TGV_primal_v_kernel on contiguous pixel ranges, where the row items
@@ -1883,8 +1912,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 &
   const int li = xcd_item(blockIdx.x, nitems);
   const int2 it = items ? items[li] : make_int2(0, li);  // null: the dense single-slice list
   const SliceDev& d = sl[it.x];
-  if constexpr (FUSED) {
-    rows_adj_fused<R, MODE, GAP, NT, NF, NEXT>(d, it.y, part_rows, smem_raw);
+  if constexpr (FUSED != 0) {
+    rows_adj_fused<R, MODE, GAP, NT, NF, FUSED, NEXT>(d, it.y, part_rows, smem_raw);
     return;
   }
   const int W = NF > 0 ? NF : d.W, H = d.H, nc = d.ncols;
@@ -2417,10 +2446,19 @@ bool fft_len_compiled(int dtype, int n) {
 bool rows_adj_fused_ok(int dtype, int W, int C, int nc) {
   constexpr int NW = kRowAdjThreadsWide;
   if (!fft_len_compiled(dtype, W) || 2 * W > NW || C < 1) return false;
-  const int ngs = std::min(NW / W, C), ch = (C + ngs - 1) / ngs;
+  const int ch = fused_coils(W, C);
   // (padded lengths: a wave holds the listed columns of its coils, 64 per slot)
   const bool cols_fit = ct_pad_ok(W) ? nc <= 64 * rows_adj_pt<NW>() : C * nc <= rows_adj_pt<NW>() * NW;
-  return ch <= kRowsAdjFusedSlots && cols_fit;
+  return ch <= (fused_more_ok(W) ? kFusedSlotsMore : kFusedSlots) && cols_fit;
+}
+
+// Calls fn with the sensitivity slots of the fused adjoint row path for C coils.
+template <int NF, class Fn>
+static void with_slots(int C, Fn&& fn) {
+  if constexpr (fused_more_ok(NF)) {
+    if (fused_coils(NF, C) > kFusedSlots) return fn(std::integral_constant<int, kFusedSlotsMore>{});
+  }
+  fn(std::integral_constant<int, kFusedSlots>{});
 }
 
 // Adjoint row pass with L.adj_threads threads per block (kRowThreads, or
@@ -2433,8 +2471,12 @@ static void launch_rows_adj(const Launch& L, bool gap) {
     const int nv = L.dense ? L.nvstep : 0;
     if constexpr (NF > 0 && MODE != M_OP) {
       if (L.adj_fused) {
-        if (gap) PDT_LAUNCH_NT((k_rows_adj<R, MODE, true, NW, NF, true>), L.nrg_a + nv, NW, lds, L.stream, L.sl, L.dense ? nullptr : L.rowgroups_a, L.nrg_a, L.cb_a, L.gap_rows, nv);
-        else PDT_LAUNCH_NT((k_rows_adj<R, MODE, false, NW, NF, true>), L.nrg_a + nv, NW, lds, L.stream, L.sl, L.dense ? nullptr : L.rowgroups_a, L.nrg_a, L.cb_a, L.gap_rows, nv);
+        const size_t lds = lds_occupancy(fused_lds(NF, L.cb_a, sizeof(Cx<R>)), L.wpc[WPC_ADJ], init_kernel_attrs());
+        with_slots<NF>(L.cb_a, [&](auto ps) {
+          constexpr int PS = decltype(ps)::value;
+          if (gap) PDT_LAUNCH_NT((k_rows_adj<R, MODE, true, NW, NF, PS>), L.nrg_a + nv, NW, lds, L.stream, L.sl, L.dense ? nullptr : L.rowgroups_a, L.nrg_a, L.cb_a, L.gap_rows, nv);
+          else PDT_LAUNCH_NT((k_rows_adj<R, MODE, false, NW, NF, PS>), L.nrg_a + nv, NW, lds, L.stream, L.sl, L.dense ? nullptr : L.rowgroups_a, L.nrg_a, L.cb_a, L.gap_rows, nv);
+        });
         return;
       }
     }
@@ -2544,11 +2586,14 @@ static void mri_pair_m(const Launch& L, int which) {
   if (which == 0) {
     launch_cols_gap<R, CM_SOLVE, GAP, MODE>(L, nullptr, L.ndual, L.part[0] + size_t(L.nrg) * kGapTerms);
   } else {
-    const size_t lds = lds_occupancy(L.lds_rows_a, L.wpc[WPC_ADJ], init_kernel_attrs());
     with_fft_len<R>(L.fft_w, [&](auto nf) {
       constexpr int NF = decltype(nf)::value;
-      if constexpr (NF > 0)
-        PDT_LAUNCH_NT((k_rows_adj<R, MODE, GAP, NW, NF, true, true>), L.nrg_a + L.nvstep, NW, lds, L.stream, L.sl, nullptr, L.nrg_a, L.cb_a, L.gap_rows, L.nvstep);
+      if constexpr (NF > 0) {
+        const size_t lds = lds_occupancy(fused_lds(NF, L.cb_a, sizeof(Cx<R>)), L.wpc[WPC_ADJ], init_kernel_attrs());
+        with_slots<NF>(L.cb_a, [&](auto ps) {
+          PDT_LAUNCH_NT((k_rows_adj<R, MODE, GAP, NW, NF, decltype(ps)::value, true>), L.nrg_a + L.nvstep, NW, lds, L.stream, L.sl, nullptr, L.nrg_a, L.cb_a, L.gap_rows, L.nvstep);
+        });
+      }
     });
   }
 }
@@ -2644,16 +2689,19 @@ static bool set_lds_attrs(int b) {
     set((const void*)&k_rows_adj<R, M_TGV, false, kRowAdjThreadsWide, NF>);
     set((const void*)&k_rows_adj<R, M_TGV, true, kRowAdjThreadsWide, NF>);
     if constexpr (NF > 0) {
-      set((const void*)&k_rows_adj<R, M_TV, false, kRowAdjThreadsWide, NF, true>);
-      set((const void*)&k_rows_adj<R, M_TV, true, kRowAdjThreadsWide, NF, true>);
-      set((const void*)&k_rows_adj<R, M_TGV, false, kRowAdjThreadsWide, NF, true>);
-      set((const void*)&k_rows_adj<R, M_TGV, true, kRowAdjThreadsWide, NF, true>);
-      if constexpr (std::is_same<R, float>::value) {
-        set((const void*)&k_rows_adj<R, M_TV, false, kRowAdjThreadsWide, NF, true, true>);
-        set((const void*)&k_rows_adj<R, M_TGV, false, kRowAdjThreadsWide, NF, true, true>);
-        set((const void*)&k_rows_adj<R, M_TV, true, kRowAdjThreadsWide, NF, true, true>);
-        set((const void*)&k_rows_adj<R, M_TGV, true, kRowAdjThreadsWide, NF, true, true>);
-      }
+      auto fused = [&](auto ps) {
+        constexpr int PS = decltype(ps)::value;
+        set((const void*)&k_rows_adj<R, M_TV, false, kRowAdjThreadsWide, NF, PS>);
+        set((const void*)&k_rows_adj<R, M_TV, true, kRowAdjThreadsWide, NF, PS>);
+        set((const void*)&k_rows_adj<R, M_TGV, false, kRowAdjThreadsWide, NF, PS>);
+        set((const void*)&k_rows_adj<R, M_TGV, true, kRowAdjThreadsWide, NF, PS>);
+        set((const void*)&k_rows_adj<R, M_TV, false, kRowAdjThreadsWide, NF, PS, true>);
+        set((const void*)&k_rows_adj<R, M_TGV, false, kRowAdjThreadsWide, NF, PS, true>);
+        set((const void*)&k_rows_adj<R, M_TV, true, kRowAdjThreadsWide, NF, PS, true>);
+        set((const void*)&k_rows_adj<R, M_TGV, true, kRowAdjThreadsWide, NF, PS, true>);
+      };
+      fused(std::integral_constant<int, kFusedSlots>{});
+      if constexpr (fused_more_ok(NF)) fused(std::integral_constant<int, kFusedSlotsMore>{});
     }
   };
   auto col = [&](auto nf) {

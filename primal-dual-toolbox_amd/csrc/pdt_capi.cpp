@@ -281,14 +281,9 @@ struct pdt_op {
   std::vector<int> h_cols;
   FftPlanD planW{}, planH{};
   // operator-mode scratch
-  DevBuf T1, T2, wpart, ctl, slice, rows, rowgroups, colitems;
-  int nrows = 0, nrg = 0, ncolitems = 0, cb = 1, cg = 1;
-  size_t lds_rows = 0, lds_cols = 0;
-  hipStream_t stream = nullptr;
-  // host source of the descriptor copy (pinned, outlives the asynchronous
-  // copy) and the completion of the last application, which shares the
-  // descriptor and the scratch planes with the next one
-  SliceDev* h_desc = nullptr;
+  DevBuf T1, T2, wpart, slice;
+  // completion of the last application, which shares the descriptor and the
+  // scratch planes with the next one
   hipEvent_t done = nullptr;
 
   int required() const { return kind == PDT_OP_SAMPLING ? 1 : 2; }
@@ -412,42 +407,6 @@ struct pdt_op {
     lc = lds_cols_bytes(dt, cg_out, Hk);
   }
 
-  void ensure_opmode() {
-    prepare();
-    if (!stream) HIPC(hipStreamCreate(&stream));
-    const size_t ce = esize(cplx_of(dtype));
-    T1.ensure(std::max<size_t>(1, size_t(C) * H * ncols * ce));
-    T2.ensure(std::max<size_t>(1, size_t(C) * H * ncols * ce));
-    if (!ctl.p) {
-      ctl.alloc(CTL_WORDS * sizeof(int));
-      int h[CTL_WORDS] = {1, 0, 0, 0, 0, 0, 0, 0};
-      HIPC(hipMemcpy(ctl.p, h, sizeof(h), hipMemcpyHostToDevice));
-    }
-    choose_tiles(cb, cg, lds_rows, lds_cols);
-    const int ngr = (C + cb - 1) / cb;
-    wpart.ensure(size_t(ngr) * H * W * ce);
-    if (!rows.p) {
-      std::vector<int2> r(H), rg;
-      for (int y = 0; y < H; ++y) r[y] = make_int2(0, y);
-      for (int y = 0; y < H; ++y)
-        for (int g = 0; g < ngr; ++g) rg.push_back(make_int2(0, y * ngr + g));
-      rows.alloc(r.size() * sizeof(int2));
-      HIPC(hipMemcpy(rows.p, r.data(), r.size() * sizeof(int2), hipMemcpyHostToDevice));
-      nrows = H;
-      rowgroups.alloc(rg.size() * sizeof(int2));
-      HIPC(hipMemcpy(rowgroups.p, rg.data(), rg.size() * sizeof(int2), hipMemcpyHostToDevice));
-      nrg = (int)rg.size();
-      const int ng = (ncols + cg - 1) / cg;
-      std::vector<int2> c;
-      for (int cc = 0; cc < C; ++cc)
-        for (int g = 0; g < ng; ++g) c.push_back(make_int2(0, cc * ng + g));
-      colitems.alloc(std::max<size_t>(1, c.size()) * sizeof(int2));
-      if (!c.empty()) HIPC(hipMemcpy(colitems.p, c.data(), c.size() * sizeof(int2), hipMemcpyHostToDevice));
-      ncolitems = (int)c.size();
-      slice.alloc(sizeof(SliceDev));
-    }
-  }
-
   SliceDev geometry() const {
     SliceDev d{};
     d.W = W;
@@ -465,75 +424,86 @@ struct pdt_op {
     return d;
   }
 
-  // Applies A (forward) or A^* (adjoint) from device src to device dst.
-  void apply(bool forward, const void* src, void* dst, hipStream_t st) {
-    SetupLock lk(g_setup_mu);
-    ensure_opmode();
-    SliceDev d = geometry();
+  // The launches of an application with the workspaces of d (T1, T2, wpart)
+  // and the descriptor's place d_dev in device memory.
+  void launch(bool forward, SliceDev d, SliceDev* d_dev, const void* src, void* dst, int cb, int cg, size_t lr, size_t lc,
+              hipStream_t st) const {
     d.ngroups = (ncols + cg - 1) / cg;
     d.ngr = (C + cb - 1) / cb;
-    d.ngr_a = d.ngr;
-    d.T1 = T1.p;
-    d.T2 = T2.p;
-    d.wpart = wpart.p;
+    const int dt = dtype == PDT_C128 ? DT_C128 : DT_C64;
+    // Adjoint: every coil of a row in one workgroup of 1024 threads where the
+    // row has a plan and work for them, which also sums the coils; else coil
+    // groups and k_mri_primal.  A and A^*: 512 x 512, 8 coils 88 us against
+    // 95; 320 x 320, 15 coils 66 against 68; 64 x 256, 8 coils 46.5 against
+    // 48.3; 256 x 256, 5 coils (below the line) 47.4 either way.
+    const size_t lra = lds_rows_bytes(dt, C, W, ncols, false);
+    const bool wide = C > cb && C * W >= 8 * kRowThreads && fft_len_compiled(dt, W) && lra <= init_kernel_attrs();
+    d.ngr_a = wide ? 1 : d.ngr;
     d.op_in = src;
     d.op_out = dst;
-    d.ctl = ctl.as<int>();
-    if (!h_desc) HIPC(hipHostMalloc((void**)&h_desc, sizeof(SliceDev), hipHostMallocDefault));
-    if (done) HIPC(hipEventSynchronize(done));  // the previous application (any stream) has finished
-    else HIPC(hipEventCreateWithFlags(&done, hipEventDisableTiming));
-    *h_desc = d;
-    HIPC(hipMemcpyAsync(slice.p, h_desc, sizeof(d), hipMemcpyHostToDevice, st));
     Launch L;
     L.stream = st;
-    L.sl = slice.as<SliceDev>();
+    L.sl = d_dev;
     L.nsl = 1;
-    L.rows = rows.as<int2>();
-    L.nrows = nrows;
-    L.rowgroups = rowgroups.as<int2>();
-    L.nrg = nrg;
-    L.cols = colitems.as<int2>();
-    L.ncolitems = ncolitems;
+    // identity lists: rows y, (row, coil group), (coil, column group)
+    L.nrows = H;
+    L.nrg = H * d.ngr;
+    L.nrg_a = H * d.ngr_a;
+    L.ncolitems = C * d.ngroups;
     L.cb = cb;
+    L.cb_a = wide ? C : cb;
     L.cg = cg;
-    L.lds_rows = lds_rows;
-    L.lds_cols = lds_cols;
+    L.lds_rows = lr;
+    L.lds_rows_a = wide ? lra : lr;
+    L.lds_cols = lc;
     L.fft_w = W;
     L.fft_h = Hk;
     L.split_primal = d.ngr_a > 1;
     L.primal_threads = primal_block(W);
-    L.rowgroups_a = L.rowgroups;
-    L.nrg_a = L.nrg;
-    L.cb_a = L.cb;
-    L.lds_rows_a = L.lds_rows;
-    L.adj_threads = kRowThreads;
-    const int dt = dtype == PDT_C128 ? DT_C128 : DT_C64;
-    if (forward) {
-      run_zero(st, dst, size_t(W) * Hk * C * esize(cplx_of(dtype)));
-      if (ncols) run_op_forward(L, dt);
-    } else {
-      if (ncols) run_op_adjoint(L, dt);
-      else run_zero(st, dst, size_t(W) * H * esize(cplx_of(dtype)));
-    }
+    L.adj_threads = wide ? kRowAdjThreadsWide : kRowThreads;
+    const size_t ce = esize(cplx_of(dtype));
+    if (ncols == 0) run_zero(st, dst, size_t(W) * (forward ? size_t(Hk) * C : size_t(H)) * ce);
+    else if (forward) run_op_forward(L, dt, d);
+    else run_op_adjoint(L, dt, d);
     HIPC(hipGetLastError());
+  }
+
+  // Applies A (forward) or A^* (adjoint) from device src to device dst.
+  void apply(bool forward, const void* src, void* dst, hipStream_t st) {
+    SetupLock lk(g_setup_mu);
+    prepare();
+    int cb = 1, cg = 1;
+    size_t lr = 0, lc = 0;
+    choose_tiles(cb, cg, lr, lc);
+    if (done) HIPC(hipEventSynchronize(done));  // the previous application (any stream) has finished
+    else HIPC(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    const size_t ce = esize(cplx_of(dtype));
+    T1.ensure(std::max<size_t>(1, size_t(C) * H * ncols * ce));
+    T2.ensure(std::max<size_t>(1, size_t(C) * H * ncols * ce));
+    wpart.ensure(size_t((C + cb - 1) / cb) * H * W * ce);
+    slice.ensure(sizeof(SliceDev));
+    SliceDev d = geometry();
+    d.T1 = T1.p;
+    d.T2 = T2.p;
+    d.wpart = wpart.p;
+    launch(forward, d, slice.as<SliceDev>(), src, dst, cb, cg, lr, lc, st);
     HIPC(hipEventRecord(done, st));
   }
 
   // apply() without any device allocation: the intermediates (descriptor,
-  // control words, T1, T2, per-group partial adjoints) live in the per-GPU
-  // scratch array, the work lists are the identity (null lists), and the
-  // descriptor is written by a kernel from its by-value argument.  Needs the
-  // prepared geometry (prepare() allocates) and enqueues on st without
-  // waiting.  Calls that overlap on one GPU share the array and race.
+  // T1, T2, per-group partial adjoints) live in the per-GPU scratch array.
+  // Needs the prepared geometry (prepare() allocates) and enqueues on st
+  // without waiting.  Calls that overlap on one GPU share the array and race.
   void apply_noalloc(bool forward, const void* src, void* dst, hipStream_t st) {
-    int cbn = 1, cgn = 1;
+    int cb = 1, cg = 1;
     size_t lr = 0, lc = 0;
-    choose_tiles(cbn, cgn, lr, lc);
+    choose_tiles(cb, cg, lr, lc);
     const size_t ce = esize(cplx_of(dtype));
-    const int ngr = (C + cbn - 1) / cbn, ng = (ncols + cgn - 1) / cgn;
+    const int ngr = (C + cb - 1) / cb;
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const size_t o_ctl = al(sizeof(SliceDev));
-    const size_t o_t1 = o_ctl + al(CTL_WORDS * sizeof(int));
+    // (the size limit counts a block of control words, which an application
+    // no longer has, after the descriptor)
+    const size_t o_t1 = al(sizeof(SliceDev)) + al(CTL_WORDS * sizeof(int));
     const size_t tb = al(size_t(C) * H * ncols * ce);
     const size_t o_t2 = o_t1 + tb, o_wp = o_t2 + tb;
     const size_t need = o_wp + (ngr > 1 ? al(size_t(ngr) * H * W * ce) : 0);
@@ -548,49 +518,10 @@ struct pdt_op {
     char* base = static_cast<char*>(noalloc_scratch(dev));
     if (!base) fail(PDT_ERR_HIP, "the scratch array of the allocation-free application is not available on this device");
     SliceDev d = geometry();
-    d.ngroups = ng;
-    d.ngr = ngr;
-    d.ngr_a = ngr;
     d.T1 = base + o_t1;
     d.T2 = base + o_t2;
     d.wpart = ngr > 1 ? base + o_wp : nullptr;
-    d.op_in = src;
-    d.op_out = dst;
-    d.ctl = reinterpret_cast<int*>(base + o_ctl);
-    SliceDev* d_dev = reinterpret_cast<SliceDev*>(base);
-    run_store_desc(st, d, d_dev, d.ctl);
-    Launch L;
-    L.stream = st;
-    L.sl = d_dev;
-    L.nsl = 1;
-    L.rows = nullptr;  // identity lists: rows y, (row, coil group), (coil, column group)
-    L.nrows = H;
-    L.rowgroups = nullptr;
-    L.nrg = H * ngr;
-    L.cols = nullptr;
-    L.ncolitems = C * ng;
-    L.cb = cbn;
-    L.cg = cgn;
-    L.lds_rows = lr;
-    L.lds_cols = lc;
-    L.fft_w = W;
-    L.fft_h = Hk;
-    L.split_primal = ngr > 1;
-    L.primal_threads = primal_block(W);
-    L.rowgroups_a = nullptr;
-    L.nrg_a = L.nrg;
-    L.cb_a = cbn;
-    L.lds_rows_a = lr;
-    L.adj_threads = kRowThreads;
-    const int dt = dtype == PDT_C128 ? DT_C128 : DT_C64;
-    if (forward) {
-      run_zero(st, dst, size_t(W) * Hk * C * ce);
-      if (ncols) run_op_forward(L, dt);
-    } else {
-      if (ncols) run_op_adjoint(L, dt);
-      else run_zero(st, dst, size_t(W) * H * ce);
-    }
-    HIPC(hipGetLastError());
+    launch(forward, d, reinterpret_cast<SliceDev*>(base), src, dst, cb, cg, lr, lc, st);
   }
 
   ~pdt_op() {
@@ -598,8 +529,6 @@ struct pdt_op {
       (void)hipEventSynchronize(done);
       (void)hipEventDestroy(done);
     }
-    if (h_desc) (void)hipHostFree(h_desc);
-    if (stream) (void)hipStreamDestroy(stream);
   }
 };
 

@@ -1147,14 +1147,22 @@ __device__ __forceinline__ void dual_workgroup(const SliceDev& d, int nd, double
 }
 
 template <class R, int MODE, bool GAP, int NT, int NF>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GAP ? 5 : 1))) void k_rows_fwd(const SliceDev* sl, const int2* items, int nitems, int cb,
-                                                 double* part, int ndual) {
-  extern __shared__ char smem_raw[];
+__device__ __forceinline__ void rows_fwd(const SliceDev* sl, const int2* items, int nitems, int cb, double* part,
+                                         int ndual, char* smem_raw) {
   using C = Cx<R>;
-  if (MODE != M_OP && int(blockIdx.x) >= nitems) {
+  if (int(blockIdx.x) >= nitems) {
     const SliceDev& d = sl[0];
-    if (!slice_active(d)) return;
-    dual_workgroup<R, MODE, GAP, NT>(d, ndual, part + size_t(nitems) * kGapTerms);
+    if constexpr (MODE == M_OP) {
+      // operator forward: the output, of which the column pass writes the
+      // listed columns only, is zeroed beside the row transforms
+      const size_t n = size_t(d.W) * d.Hk * d.C, chunk = (n + ndual - 1) / ndual;
+      const size_t b = size_t(blockIdx.x - nitems) * chunk, e = min(n, b + chunk);
+      const auto out = gptr<C>(d.op_out);
+      for (size_t i = b + threadIdx.x; i < e; i += NT) out[i] = pzero<C>();
+    } else {
+      if (!slice_active(d)) return;
+      dual_workgroup<R, MODE, GAP, NT>(d, ndual, part + size_t(nitems) * kGapTerms);
+    }
     return;
   }
   const int li = xcd_item(blockIdx.x, nitems);
@@ -1205,7 +1213,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GAP ? 5 : 1)
   }
   // A finished slice's blocks leave before their first store; the check comes
   // after the loads above are issued, so its control-word load overlaps them.
-  if (!slice_active(d)) return;
+  if (MODE != M_OP && !slice_active(d)) return;
   double t[kGapTerms] = {0};
   if (MODE != M_OP && ndual == 0) {
     // The dual step of row y is shared out over the row's coil groups in
@@ -1245,6 +1253,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GAP ? 5 : 1)
   if (GAP) block_sum<3, NT>(reinterpret_cast<double(&)[3]>(t), part + size_t(li) * kGapTerms);
 }
 
+template <class R, int MODE, bool GAP, int NT, int NF>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(GAP ? 5 : 1))) void k_rows_fwd(const SliceDev* sl, const int2* items, int nitems, int cb,
+                                                 double* part, int ndual) {
+  extern __shared__ char smem_raw[];
+  rows_fwd<R, MODE, GAP, NT, NF>(sl, items, nitems, cb, part, ndual, smem_raw);
+}
+
+// The first launch of an operator application takes its descriptor by value
+// and leaves it in memory for the launches after it (a launch or a copy less
+// in front of it: 3.2 us and its gap).
+__device__ __forceinline__ void store_desc(const SliceDev& d, SliceDev* dst) {
+  static_assert(sizeof(SliceDev) % 8 == 0, "whole words");
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < int(sizeof(SliceDev) / 8); i += blockDim.x)
+      reinterpret_cast<uint64_t*>(dst)[i] = reinterpret_cast<const uint64_t*>(&d)[i];
+}
+template <class R, int NT, int NF>
+__global__ __launch_bounds__(NT) void k_op_rows_fwd(const SliceDev d, SliceDev* dst, int nitems, int cb, int nzero) {
+  extern __shared__ char smem_raw[];
+  store_desc(d, dst);
+  rows_fwd<R, M_OP, false, NT, NF>(&d, nullptr, nitems, cb, nullptr, nzero, smem_raw);
+}
+
 // Column pass.  CMODE: 0 solver (forward, r prox, adjoint), 1 operator
 // forward (writes op_out {W, Hk, C}), 2 operator adjoint (reads op_in).
 // PF (solver, compile-time length, at most kColPrefetchCols columns per
@@ -1259,12 +1290,11 @@ enum { CM_SOLVE = 0, CM_FWD = 1, CM_ADJ = 2 };
 // to part_dual), which reads and writes none of what the column items do;
 // with the adjoint row pass also writing the next T1 (k_rows_adj NEXT) an
 // iteration is these two launches.
-template <class R, int CMODE, bool GAP, int NT, int NF, bool PF = false, int DUAL = 0>
-__global__ __launch_bounds__(NT) void k_cols(const SliceDev* sl, const int2* items, int nitems, int cg,
-                                             double* part, int ndual, double* part_dual) {
+template <class R, int CMODE, bool GAP, int NT, int NF, bool PF, int DUAL>
+__device__ __forceinline__ void cols(const SliceDev* sl, const int2* items, int nitems, int cg, double* part, int ndual,
+                                     double* part_dual, char* smem_raw) {
   static_assert(!PF || (NF > 0 && CMODE == CM_SOLVE), "register prefetch needs a compile-time length");
   static_assert(DUAL == 0 || CMODE == CM_SOLVE, "dual workgroups: solver iterations");
-  extern __shared__ char smem_raw[];
   if (DUAL != 0 && int(blockIdx.x) >= nitems) {
     const SliceDev& d = sl[0];
     if (!slice_active(d)) return;
@@ -1328,7 +1358,7 @@ __global__ __launch_bounds__(NT) void k_cols(const SliceDev* sl, const int2* ite
       pf_m[k] = mk[e];
     }
   }
-  if (!slice_active(d)) return;  // after the loads are issued, before any store
+  if (CMODE == CM_SOLVE && !slice_active(d)) return;  // after the loads are issued, before any store
   if (CMODE != CM_ADJ) {
     // registers -> LDS with the prefetch, else the gather straight into LDS
     if (pf) {
@@ -1404,6 +1434,19 @@ __global__ __launch_bounds__(NT) void k_cols(const SliceDev* sl, const int2* ite
   if (GAP) block_sum<2, NT>(t, part + size_t(li) * kGapTerms);
 }
 
+template <class R, int CMODE, bool GAP, int NT, int NF, bool PF = false, int DUAL = 0>
+__global__ __launch_bounds__(NT) void k_cols(const SliceDev* sl, const int2* items, int nitems, int cg,
+                                             double* part, int ndual, double* part_dual) {
+  extern __shared__ char smem_raw[];
+  cols<R, CMODE, GAP, NT, NF, PF, DUAL>(sl, items, nitems, cg, part, ndual, part_dual, smem_raw);
+}
+template <class R, int NT, int NF>
+__global__ __launch_bounds__(NT) void k_op_cols_adj(const SliceDev d, SliceDev* dst, int nitems, int cg) {
+  extern __shared__ char smem_raw[];
+  store_desc(d, dst);
+  cols<R, CM_ADJ, false, NT, NF, false, 0>(&d, nullptr, nitems, cg, nullptr, 0, nullptr, smem_raw);
+}
+
 // Column pass of the lengths 8 M 8 (with_direct_cols): a thread does one
 // butterfly of every stage, and what comes before the first stage, between the
 // two transforms and after the last one stays in its registers.  The first
@@ -1428,15 +1471,13 @@ struct ColShape {
   static constexpr int NP = NF + NF / 8;          // LDS slots of a column, one pad slot per 8 elements
   static constexpr size_t lds = (NF + 2 * size_t(CS) * NP) * sizeof(Cx<R>);
 };
-template <class R, int CMODE, bool GAP, int NF, int DUAL = 0>
-__global__ __launch_bounds__((ColShape<R, NF>::NT)) void k_cols_direct(const SliceDev* sl, const int2* items, int nitems,
-                                                                     int cg, double* part, int ndual,
-                                                                     double* part_dual) {
+template <class R, int CMODE, bool GAP, int NF, int DUAL>
+__device__ __forceinline__ void cols_direct(const SliceDev* sl, const int2* items, int nitems, int cg, double* part,
+                                            int ndual, double* part_dual, char* smem_raw) {
   using C = Cx<R>;
   using Sh = ColShape<R, NF>;
   constexpr int CS = Sh::CS, M = Sh::M, NR = Sh::NR, NT = Sh::NT, NP = Sh::NP, NRP = NR + NR / 8, Hk = NF;
   static_assert(NF == 64 * M && NR % 8 == 0, "8 M 8, padded");
-  extern __shared__ char smem_raw[];
   if (DUAL != 0 && int(blockIdx.x) >= nitems) {
     const SliceDev& d = sl[0];
     if (!slice_active(d)) return;
@@ -1518,7 +1559,7 @@ __global__ __launch_bounds__((ColShape<R, NF>::NT)) void k_cols_direct(const Sli
       pf[q] = in[size_t((actp ? ip : 0) + kfe(0, q)) * W + col];
     }
   }
-  if (!slice_active(d)) return;  // after the loads are issued, before any store
+  if (CMODE == CM_SOLVE && !slice_active(d)) return;  // after the loads are issued, before any store
   s_tw.store(tw, Hk);
   if (CMODE != CM_ADJ) {
     // forward: 8, M, 8
@@ -1584,6 +1625,21 @@ __global__ __launch_bounds__((ColShape<R, NF>::NT)) void k_cols_direct(const Sli
     }
   }
   if (GAP) block_sum<2, NT>(t, part + size_t(li) * kGapTerms);
+}
+
+template <class R, int CMODE, bool GAP, int NF, int DUAL = 0>
+__global__ __launch_bounds__((ColShape<R, NF>::NT)) void k_cols_direct(const SliceDev* sl, const int2* items, int nitems,
+                                                                     int cg, double* part, int ndual,
+                                                                     double* part_dual) {
+  extern __shared__ char smem_raw[];
+  cols_direct<R, CMODE, GAP, NF, DUAL>(sl, items, nitems, cg, part, ndual, part_dual, smem_raw);
+}
+template <class R, int NF>
+__global__ __launch_bounds__((ColShape<R, NF>::NT)) void k_op_cols_adj_direct(const SliceDev d, SliceDev* dst, int nitems,
+                                                                            int cg) {
+  extern __shared__ char smem_raw[];
+  store_desc(d, dst);
+  cols_direct<R, CM_ADJ, false, NF, 0>(&d, nullptr, nitems, cg, nullptr, 0, nullptr, smem_raw);
 }
 
 // Primal step of pixel (x, y) given w = (A^* r)(x, y):
@@ -1982,7 +2038,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 &
   } else {
     copy_to_lds<int, NF, NT>(L.cols, gcols, nc);
   }
-  if (!slice_active(d)) return;  // after the loads above are issued, before any store
+  if (MODE != M_OP && !slice_active(d)) return;  // after the loads above are issued, before any store
   // With all coils of the row in one block of at least 2 W threads, the
   // parts of the primal step that do not need A^* r run before the FFT, so
   // their loads overlap those of S and T2: threads x < W load u(x, y) and
@@ -2106,7 +2162,7 @@ __global__ __launch_bounds__(1024) void k_mri_primal(const SliceDev* sl, const i
   const int li = xcd_item(blockIdx.x, nitems);
   const int2 it = items ? items[li] : make_int2(0, li * rpi);  // null: the dense single-slice list
   const SliceDev& d = sl[it.x];
-  if (!slice_active(d) || d.ngr_a == 1) return;
+  if ((MODE != M_OP && !slice_active(d)) || d.ngr_a == 1) return;
   using C = Cx<R>;
   const int W = d.W, H = d.H, ngr = d.ngr_a;
   const size_t n = size_t(W) * H;
@@ -2289,14 +2345,6 @@ __global__ __launch_bounds__(kBlock) void k_compact(const SliceDev* sl, const in
     }
   }
   block_sum<1>(t, part + size_t(blockIdx.x) * kGapTerms);
-}
-
-// Writes a slice descriptor passed by value to device memory and opens its
-// control words (active, iteration 0): the set-up of an operator application
-// that copies nothing from the host.
-__global__ __launch_bounds__(64) void k_store_desc(SliceDev d, SliceDev* dst, int* ctl) {
-  if (threadIdx.x == 0) *dst = d;
-  if (threadIdx.x < CTL_WORDS) ctl[threadIdx.x] = threadIdx.x == CTL_ACTIVE ? 1 : 0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_zero(uint32_t* p, size_t n) {
@@ -2505,7 +2553,7 @@ int default_cg(int Hk) {
 
 // Column pass (DUAL: with the dual step's workgroups, gap terms to pd).
 template <class R, int CMODE, bool GAP, int DUAL>
-static void launch_cols_gap(const Launch& L, const int2* items, int ndual, double* pd) {
+static void launch_cols(const Launch& L, const int2* items, int ndual, double* pd) {
   constexpr int NC = kColThreads;
   const size_t limit = init_kernel_attrs();
   bool done = false;
@@ -2529,17 +2577,6 @@ static void launch_cols_gap(const Launch& L, const int2* items, int ndual, doubl
     PDT_LAUNCH_NT((k_cols<R, CMODE, GAP, NC, NF, false, DUAL>), L.ncolitems + ndual, NC, lds, L.stream, L.sl, items, L.ncolitems, L.cg, L.part[1], ndual, pd);
   });
 }
-template <class R, int CMODE>
-static void launch_cols(const Launch& L, bool gap, const int2* items) {
-  if constexpr (CMODE == CM_SOLVE) {
-    if (gap) {
-      launch_cols_gap<R, CMODE, true, 0>(L, items, 0, nullptr);
-      return;
-    }
-  }
-  launch_cols_gap<R, CMODE, false, 0>(L, items, 0, nullptr);
-}
-
 // MRI stages: 0 rows_fwd, 1 cols, 2 rows_adj, 3 primal.  The FFT kernels are
 // picked by L.fft_w (row length) and L.fft_h (column length).
 template <class R, int MODE>
@@ -2555,7 +2592,9 @@ static void mri_stage_m(const Launch& L, bool gap, int stage) {
     });
   } else if (stage == 1) {
     if (L.ncolitems == 0) return;
-    launch_cols<R, CM_SOLVE>(L, gap, L.dense ? nullptr : L.cols);
+    const int2* items = L.dense ? nullptr : L.cols;
+    if (gap) launch_cols<R, CM_SOLVE, true, 0>(L, items, 0, nullptr);
+    else launch_cols<R, CM_SOLVE, false, 0>(L, items, 0, nullptr);
   } else if (stage == 2) {
     with_fft_len<R>(L.fft_w, [&](auto nf) {
       constexpr int NF = decltype(nf)::value;
@@ -2584,7 +2623,7 @@ template <class R, int MODE, bool GAP>
 static void mri_pair_m(const Launch& L, int which) {
   constexpr int NW = kRowAdjThreadsWide;
   if (which == 0) {
-    launch_cols_gap<R, CM_SOLVE, GAP, MODE>(L, nullptr, L.ndual, L.part[0] + size_t(L.nrg) * kGapTerms);
+    launch_cols<R, CM_SOLVE, GAP, MODE>(L, nullptr, L.ndual, L.part[0] + size_t(L.nrg) * kGapTerms);
   } else {
     with_fft_len<R>(L.fft_w, [&](auto nf) {
       constexpr int NF = decltype(nf)::value;
@@ -2643,18 +2682,32 @@ void run_gap_reduce(const Launch& L, int kind, int dtype) {
 }
 
 template <class R>
-static void op_forward(const Launch& L) {
+static void op_forward(const Launch& L, const SliceDev& d) {
   constexpr int NR = kRowThreads;
+  SliceDev* const dst = const_cast<SliceDev*>(L.sl);
+  // zeroing workgroups: 32 elements per thread
+  const int nz = int((int64_t(d.W) * d.Hk * d.C + 32 * NR - 1) / (32 * NR));
   with_fft_len<R>(L.fft_w, [&](auto nf) {
-    constexpr int NF = decltype(nf)::value;
-    PDT_LAUNCH_NT((k_rows_fwd<R, M_OP, false, NR, NF>), L.nrg, NR, L.lds_rows, L.stream, L.sl, L.rowgroups, L.nrg, L.cb, L.part[0], 0);
+    PDT_LAUNCH_NT((k_op_rows_fwd<R, NR, decltype(nf)::value>), L.nrg + nz, NR, L.lds_rows, L.stream, d, dst, L.nrg, L.cb, nz);
   });
-  launch_cols<R, CM_FWD>(L, false, L.cols);
+  launch_cols<R, CM_FWD, false, 0>(L, nullptr, 0, nullptr);
 }
 
 template <class R>
-static void op_adjoint(const Launch& L) {
-  launch_cols<R, CM_ADJ>(L, false, L.cols);
+static void op_adjoint(const Launch& L, const SliceDev& d) {
+  SliceDev* const dst = const_cast<SliceDev*>(L.sl);
+  bool done = false;
+  with_direct_cols(L.fft_h, [&](auto nf) {
+    constexpr int NF = decltype(nf)::value;
+    using Sh = ColShape<R, NF>;
+    if (Sh::lds > init_kernel_attrs()) return;
+    done = true;
+    PDT_LAUNCH_NT((k_op_cols_adj_direct<R, NF>), L.ncolitems, Sh::NT, Sh::lds, L.stream, d, dst, L.ncolitems, L.cg);
+  });
+  if (!done)
+    with_other_len<R>(L.fft_h, [&](auto nf) {
+      PDT_LAUNCH_NT((k_op_cols_adj<R, kColThreads, decltype(nf)::value>), L.ncolitems, kColThreads, L.lds_cols, L.stream, d, dst, L.ncolitems, L.cg);
+    });
   with_fft_len<R>(L.fft_w, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     launch_rows_adj<R, M_OP, NF>(L, false);
@@ -2673,7 +2726,7 @@ static bool set_lds_attrs(int b) {
   };
   auto one = [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
-    set((const void*)&k_rows_fwd<R, M_OP, false, NR, NF>);
+    set((const void*)&k_op_rows_fwd<R, NR, NF>);
     set((const void*)&k_rows_fwd<R, M_TV, false, NR, NF>);
     set((const void*)&k_rows_fwd<R, M_TV, true, NR, NF>);
     set((const void*)&k_rows_fwd<R, M_TGV, false, NR, NF>);
@@ -2709,7 +2762,7 @@ static bool set_lds_attrs(int b) {
     set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF>);
     set((const void*)&k_cols<R, CM_SOLVE, true, NC, NF>);
     set((const void*)&k_cols<R, CM_FWD, false, NC, NF>);
-    set((const void*)&k_cols<R, CM_ADJ, false, NC, NF>);
+    set((const void*)&k_op_cols_adj<R, NC, NF>);
     if constexpr (std::is_same<R, float>::value) {
       set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, false, M_TV>);
       set((const void*)&k_cols<R, CM_SOLVE, false, NC, NF, false, M_TGV>);
@@ -2730,7 +2783,7 @@ static bool set_lds_attrs(int b) {
     set((const void*)&k_cols_direct<R, CM_SOLVE, false, NF>);
     set((const void*)&k_cols_direct<R, CM_SOLVE, true, NF>);
     set((const void*)&k_cols_direct<R, CM_FWD, false, NF>);
-    set((const void*)&k_cols_direct<R, CM_ADJ, false, NF>);
+    set((const void*)&k_op_cols_adj_direct<R, NF>);
     if constexpr (std::is_same<R, float>::value) {
       set((const void*)&k_cols_direct<R, CM_SOLVE, false, NF, M_TV>);
       set((const void*)&k_cols_direct<R, CM_SOLVE, false, NF, M_TGV>);
@@ -2762,14 +2815,14 @@ size_t init_kernel_attrs() {
   return budget;
 }
 
-void run_op_forward(const Launch& L, int dtype) {
-  if (dtype == DT_C64) op_forward<float>(L);
-  else op_forward<double>(L);
+void run_op_forward(const Launch& L, int dtype, const SliceDev& d) {
+  if (dtype == DT_C64) op_forward<float>(L, d);
+  else op_forward<double>(L, d);
 }
 
-void run_op_adjoint(const Launch& L, int dtype) {
-  if (dtype == DT_C64) op_adjoint<float>(L);
-  else op_adjoint<double>(L);
+void run_op_adjoint(const Launch& L, int dtype, const SliceDev& d) {
+  if (dtype == DT_C64) op_adjoint<float>(L, d);
+  else op_adjoint<double>(L, d);
 }
 
 int run_compact_data(const Launch& L, int dtype, const void* f_full, double* f0_part) {
@@ -2831,10 +2884,6 @@ void run_sum_strided(hipStream_t st, const double* a, int n, int stride, double*
 void run_sumsq(hipStream_t st, int dtype, const void* z, int64_t n, double* out) {
   if (dtype == DT_C128) PDT_LAUNCH_NT((k_sumsq<double>), 1, 1024, 0, st, static_cast<const Cx<double>*>(z), n, out);
   else PDT_LAUNCH_NT((k_sumsq<float>), 1, 1024, 0, st, static_cast<const Cx<float>*>(z), n, out);
-}
-
-void run_store_desc(hipStream_t st, const SliceDev& d, SliceDev* dst, int* ctl) {
-  hipLaunchKernelGGL(k_store_desc, dim3(1), dim3(64), 0, st, d, dst, ctl);
 }
 
 // Scratch of the allocation-free operator application: one array per GPU,

@@ -119,17 +119,14 @@ constexpr int kBlockRows = 4;  // rows per wave
 void run_block(const Launch& L, const SliceDev& d, int kind, int dtype, bool fp16, int dir, int k);
 // Gap evaluation from the partial sums of the last iteration (one block/slice).
 void run_gap_reduce(const Launch& L, int kind, int dtype);
-// Operator application in operator mode (op_in -> op_out of every slice).
-void run_op_forward(const Launch& L, int dtype);
-void run_op_adjoint(const Launch& L, int dtype);
+// Operator application (d.op_in -> d.op_out) of the one slice d, which the
+// first launch leaves at L.sl for the others; the work lists are the identity.
+void run_op_forward(const Launch& L, int dtype, const SliceDev& d);
+void run_op_adjoint(const Launch& L, int dtype, const SliceDev& d);
 // Gathers full-layout data {W, Hk, C} into the compact [c][ks][kfe] layout,
 // zeroes r, and writes per-block partial sums of |f|^2 over columns without
 // samples into f0_part (nblocks entries, returned).
 int run_compact_data(const Launch& L, int dtype, const void* f_full, double* f0_part);
-// Writes slice descriptor d to dst and opens its control words ctl (a
-// kernel: nothing is copied from the host).
-void run_store_desc(hipStream_t st, const SliceDev& d, SliceDev* dst, int* ctl);
-
 // Bytes of the per-GPU scratch array of the allocation-free operator
 // application, and the largest device index it serves.
 constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;

@@ -205,9 +205,36 @@ int max_cb(int dt, int W, int nc, int C) {
   while (cb > 1 && lds_rows_bytes(dt, cb, W, nc) > init_kernel_attrs()) --cb;
   return cb;
 }
-// Default tiles before any autotuning: 4 coils per row item (columns per
-// column group: default_cg; temporally blocked denoising: block_choose).
-constexpr int kDefaultCb = 4;
+// Default tiles before any autotuning: coils per row item (columns per column
+// group: default_cg; temporally blocked denoising: block_choose).  Single
+// slices on rows without a compile-time plan take 2, in single precision and
+// wherever all_coils holds: 350 x 400, 16 coils 81 us per iteration against 88
+// with 4; in double 256 x 256, 8 coils 27.0 against 27.8, but 320 x 320, 15
+// coils 74 against 73.
+constexpr int kDefaultCb = 4, kDefaultCbPlain = 2;
+
+// Whether a single slice's adjoint row pass holds every coil of a row in one
+// workgroup by default (no coil sums through memory, no k_mri_primal): where
+// the straight-line path fits, which also makes paired iterations (256 x 256,
+// 2 coils 16.6 us per iteration against 19.3, 6 coils 18.2 against 23.4; 320 x
+// 320, 6 coils 22.8 against 29.1), and on rows without a compile-time plan
+// while two workgroups fit the LDS of a CU (217 x 230, 8 coils 36.9 against
+// 43.3; double, 256 x 256, 8 coils 27.0 against 30.5; with one workgroup per
+// CU, double 320 x 320, 8 coils it would be 52.3 against 48.9).
+bool all_coils(int dt, int W, int C, int nc) {
+  if (fft_len_compiled(dt, W)) return rows_adj_fused_ok(dt, W, C, nc);
+  return lds_rows_bytes(dt, C, W, nc, false) <= kLdsMax / 2 - 2048;
+}
+
+// Whether the adjoint row pass takes workgroups of 1024 threads: with work for
+// them in an item, or where a single slice's item holds every coil: on rows
+// without a plan from 1024 elements (217 x 230, 8 coils 36.9 us per iteration
+// against 44.4 with 256 threads), on the straight-line path always.
+bool adj_wide(bool one, int dt, int cb_a, const SliceDev& d) {
+  if (cb_a * d.W >= 8 * kRowThreads) return true;
+  if (!one || !d.S || cb_a < d.C) return false;
+  return fft_len_compiled(dt, d.W) ? rows_adj_fused_ok(dt, d.W, d.C, d.ncols) : d.C > 1 && cb_a * d.W >= 4 * kRowThreads;
+}
 
 }  // namespace
 
@@ -747,7 +774,7 @@ struct Engine {
   bool fp16 = false;
   bool pair_duals = true;  // TGV denoising: the dual step as 2-pixel vectors (even widths)
   int force_dpx = 0;       // dual step pixels per thread (0: cache / default)
-  int force_cb = 0, force_cg = 0, force_rpi = 0, force_cb_a = 0;  // autotuner overrides (0: cache / default; cg, cb_a -1: default)
+  int force_cb = 0, force_cg = 0, force_rpi = 0, force_cb_a = 0;  // autotuner overrides (0: cache / default; cb, cg, cb_a -1: default)
   int force_wpc[4] = {-1, -1, -1, -1};  // occupancy caps (-1: cache; 0: none)
   int force_tb[3] = {0, 0, -1};         // blocked ROF tiles (tb[2] -1: cache / default; 0: off)
   int force_unpaired = -1;              // MRI: 1 three launches per iteration, 0 pairs where possible (-1: cache)
@@ -829,14 +856,12 @@ struct Engine {
       TuneVal tv = tune_lookup(key);
       for (int i = 0; i < 4; ++i) L.wpc[i] = force_wpc[i] >= 0 ? force_wpc[i] : tv.wpc[i];
       unpaired = force_unpaired >= 0 ? force_unpaired != 0 : tv.unpaired != 0;
-      cb = force_cb > 0 ? force_cb : tv.cb > 0 ? tv.cb : kDefaultCb;
+      const bool one_group = ns == 1 && sv[0]->op->kind != PDT_OP_SAMPLING && all_coils(dt, maxW, maxC, maxNc);
+      const bool plain = ns == 1 && !fft_len_compiled(dt, maxW) && (one_group || dt == DT_C64);
+      const int cb_def = plain ? kDefaultCbPlain : kDefaultCb;
+      cb = force_cb > 0 ? force_cb : force_cb < 0 ? cb_def : tv.cb > 0 ? tv.cb : cb_def;
       cg = force_cg > 0 ? force_cg : force_cg < 0 ? cg_def : tv.cg > 0 ? tv.cg : cg_def;
-      // default adjoint grouping: every coil of a row in one wide block where
-      // a single slice's straight-line adjoint path fits (with the u and v
-      // steps in that pass and, by default, paired iterations), else cb
-      const bool fused_fits = ns == 1 && sv[0]->op->kind != PDT_OP_SAMPLING &&
-                              maxC * maxW >= 8 * kRowThreads && rows_adj_fused_ok(dt, maxW, maxC, maxNc);
-      const int def_cb_a = fused_fits ? maxC : cb;
+      const int def_cb_a = one_group ? maxC : cb;
       cb_a = force_cb_a > 0 ? force_cb_a : force_cb_a < 0 ? def_cb_a : tv.cb_a > 0 ? tv.cb_a : def_cb_a;
       cb = std::max(1, std::min(cb, max_cb(dt, maxW, maxNc, maxC)));
       cb_a = std::max(1, std::min(cb_a, max_cb(dt, maxW, maxNc, maxC)));
@@ -1091,7 +1116,7 @@ struct Engine {
     // adjoint blocks, a compile-time FFT length, two threads per pixel of a
     // row, one adjoint coil group)
     const bool tgv = kind == PDT_SOLVER_TGV_MRI || kind == PDT_SOLVER_TGV_OP;
-    const int nvstep = dense && sv[0]->is_op() && tgv && L.cb_a * hs[0].W >= 8 * kRowThreads &&
+    const int nvstep = dense && sv[0]->is_op() && tgv && adj_wide(one, dtk(), L.cb_a, hs[0]) &&
                                fft_len_compiled(dtk(), hs[0].W) && 2 * hs[0].W <= kRowAdjThreadsWide &&
                                hs[0].ngr_a == 1
                            ? vstep_groups(hs[0])
@@ -1132,7 +1157,7 @@ struct Engine {
         x.lds_rows = lds_rows_bytes(dt, x.cb, d0.W, nc);
         x.lds_cols = lds_cols_bytes(dt, x.cg, d0.Hk);
         // wide blocks for the adjoint pass when an item holds many coil rows
-        x.adj_threads = x.cb_a * d0.W >= 8 * kRowThreads ? kRowAdjThreadsWide : kRowThreads;
+        x.adj_threads = adj_wide(one, dt, x.cb_a, d0) ? kRowAdjThreadsWide : kRowThreads;
         x.lds_rows_a = lds_rows_bytes(dt, x.cb_a, d0.W, nc, x.adj_threads != kRowAdjThreadsWide);
       } else {
         // one thread per pixel of an item where the workgroup size allows
@@ -2450,8 +2475,8 @@ int pdt_set_tiles(pdt_solver** solvers, int count, const pdt_tiles* t) {
     e.sv = sv;
     e.plan_only = true;
     // zero or negative: the default, not a cached choice
-    e.force_cb = t->cb > 0 ? t->cb : kDefaultCb;
-    e.force_cg = t->cg > 0 ? t->cg : -1;  // (-1: the engine's default)
+    e.force_cb = t->cb > 0 ? t->cb : -1;  // (-1: the engine's default)
+    e.force_cg = t->cg > 0 ? t->cg : -1;
     e.force_rpi = t->rpi > 0 ? t->rpi : 1;
     e.force_cb_a = t->cb_a > 0 ? t->cb_a : -1;  // (-1: the engine's default grouping)
     for (int i = 0; i < 4; ++i) e.force_wpc[i] = std::max(0, std::min(t->wpc[i], 6));

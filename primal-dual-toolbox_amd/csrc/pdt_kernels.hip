@@ -2494,6 +2494,9 @@ bool fft_len_compiled(int dtype, int n) {
 bool rows_adj_fused_ok(int dtype, int W, int C, int nc) {
   constexpr int NW = kRowAdjThreadsWide;
   if (!fft_len_compiled(dtype, W) || 2 * W > NW || C < 1) return false;
+  // (unpadded lengths run their stages workgroup-wide, which takes work for
+  // 1024 threads: 368 x 368, 3 coils 34.9 us per iteration this way, 32.8 not)
+  if (!ct_pad_ok(W) && C * W < 8 * kRowThreads) return false;
   const int ch = fused_coils(W, C);
   // (padded lengths: a wave holds the listed columns of its coils, 64 per slot)
   const bool cols_fit = ct_pad_ok(W) ? nc <= 64 * rows_adj_pt<NW>() : C * nc <= rows_adj_pt<NW>() * NW;

@@ -2435,8 +2435,9 @@ static void denoise_stage(const Launch& L, int kind, bool gap, int stage) {
 #define PDT_LAUNCH_NT(kern, grid, nt, lds, st, ...) \
   hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), lds, st, __VA_ARGS__)
 
-// FFT lengths with kernels built on a compile-time plan (single precision);
-// any other length, and every double-precision launch, uses the runtime plan.
+// FFT lengths with kernels built on a compile-time plan (single precision; in
+// double precision only the column pass of with_direct_cols); any other launch
+// uses the runtime plan.
 constexpr int kFftLengths[] = {256, 320, 368, 384, 512, 640, 736, 768};
 
 // Calls fn(std::integral_constant<int, NF>) with NF = n when n has a

@@ -142,8 +142,8 @@ void run_sum_strided(hipStream_t st, const double* a, int n, int stride, double*
 // out[0] = sum of |z_i|^2 over n complex pixels (DT_C64 or DT_C128).
 void run_sumsq(hipStream_t st, int dtype, const void* z, int64_t n, double* out);
 
-// True when the row/column kernels of this precision have a compile-time
-// FFT plan for length n (the kernels fall back to the runtime plan otherwise).
+// True when the row kernels of this precision have a compile-time FFT plan for
+// length n (they fall back to the runtime plan otherwise).
 bool fft_len_compiled(int dtype, int n);
 // Whether the straight-line adjoint row path fits a slice with rows of W
 // pixels, C coils (all in one coil group) and nc listed PE columns.

@@ -1066,12 +1066,13 @@ template <class T, int NF, int NT>
 struct Staged {
   static constexpr int K = NF > 0 ? (NF + NT - 1) / NT : 1;
   T v[K];
-  // branch-free (lanes past n load element n - 1, never stored), so that the
-  // compiler's waits count these loads exactly
+  // branch-free (lanes past n load element n - 1, never stored; of an empty
+  // array, the element every buffer holds), so that the compiler's waits count
+  // these loads exactly
   template <class A>
   __device__ __forceinline__ void load(A* src, int n) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = src[min(int(threadIdx.x) + k * NT, n - 1)];
+    for (int k = 0; k < K; ++k) v[k] = src[min(int(threadIdx.x) + k * NT, max(n - 1, 0))];
   }
   __device__ __forceinline__ void store(T* dst, int n) const {
 #pragma unroll
@@ -1739,17 +1740,17 @@ __device__ __forceinline__ void rows_adj_fused(const SliceDev& d, int y, double*
   const float rnc = 1.0f / float(max(nc, 1));
   const auto T2 = gptr<const C>(d.T2) + size_t(y) * nc;
   const auto gcols = gptr<const int>(d.cols);
-  const int cstride = H * nc;
+  const int cstride = H * nc, last = max(nc - 1, 0);
   C pT[IP ? SPW : 1][PT];
   int pK[PT];
   if constexpr (IP) {
 #pragma unroll
-    for (int k = 0; k < PT; ++k) pK[k] = at(gcols, uint32_t(min(lane + 64 * k, nc - 1)));
+    for (int k = 0; k < PT; ++k) pK[k] = at(gcols, uint32_t(min(lane + 64 * k, last)));
 #pragma unroll
     for (int sq = 0; sq < SPW; ++sq)
 #pragma unroll
       for (int k = 0; k < PT; ++k)
-        pT[sq][k] = at(T2 + min(wave + NW * sq, ncb - 1) * cstride, uint32_t(min(lane + 64 * k, nc - 1)));
+        pT[sq][k] = at(T2 + min(wave + NW * sq, ncb - 1) * cstride, uint32_t(min(lane + 64 * k, last)));
   } else {
 #pragma unroll
     for (int k = 0; k < PT; ++k) {
@@ -2494,7 +2495,8 @@ bool fft_len_compiled(int dtype, int n) {
 
 bool rows_adj_fused_ok(int dtype, int W, int C, int nc) {
   constexpr int NW = kRowAdjThreadsWide;
-  if (!fft_len_compiled(dtype, W) || 2 * W > NW || C < 1) return false;
+  // (a mask without listed columns has no T2 row to hold in registers)
+  if (!fft_len_compiled(dtype, W) || 2 * W > NW || C < 1 || nc < 1) return false;
   // (unpadded lengths run their stages workgroup-wide, which takes work for
   // 1024 threads: 368 x 368, 3 coils 34.9 us per iteration this way, 32.8 not)
   if (!ct_pad_ok(W) && C * W < 8 * kRowThreads) return false;

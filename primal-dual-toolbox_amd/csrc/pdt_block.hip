@@ -104,7 +104,9 @@ struct BlockArgs {
 // their storage type after every dual step, so the iterates equal theirs bit
 // for bit.  TGV launches do not store ubar and vbar: the primal step, which
 // comes first, rewrites them.
-template <class P, class S, bool TGV, int J, bool FLAT>
+//
+// ANY: projection radii of any size (ball_any).
+template <class P, class S, bool TGV, int J, bool FLAT, bool ANY>
 __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
   using R = typename RealOf<P>::T;
   using L = Ld<P, S>;
@@ -169,7 +171,11 @@ __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
     }
   };
   const R sigma = R(d.sigma), tau = R(d.tau), lambda = R(d.lambda), theta = R(d.theta);
-  const R w0 = ball_weight(R(TGV ? d.alpha0 : 1.0)), w1 = ball_weight(R(TGV ? d.alpha1 : 1.0));
+  auto ball = [](R alpha) {
+    if constexpr (ANY) return ball_any(alpha);
+    else return ball_weight(alpha);
+  };
+  const auto w0 = ball(R(TGV ? d.alpha0 : 1.0)), w1 = ball(R(TGV ? d.alpha1 : 1.0));
   const R un_scale = rcp(R(1) + tau * lambda);
   const bool xlast = x >= W - 1, xcut = xlast && W > 1;  // (W = 1: column 0 keeps its value in a backward difference)
   // row H - 1: FLAT by its number, else the last wave's last row.  (Without a
@@ -295,12 +301,12 @@ __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
   if (blockIdx.x == 0 && threadIdx.x == 0) gptr<int>(d.ctl)[CTL_ITER] += k;
 }
 
-template <class P, class S, bool TGV, int J, int NT>
+template <class P, class S, bool TGV, int J, int NT, bool ANY>
 __global__ __launch_bounds__(NT) void k_den_block(BlockArgs d) {
   extern __shared__ char smem_raw[];
   P* const smem = reinterpret_cast<P*>(smem_raw);
-  if (int(blockDim.x >> 6) * J > d.H) block_iterations<P, S, TGV, J, true>(d, smem);
-  else block_iterations<P, S, TGV, J, false>(d, smem);
+  if (int(blockDim.x >> 6) * J > d.H) block_iterations<P, S, TGV, J, true, ANY>(d, smem);
+  else block_iterations<P, S, TGV, J, false, ANY>(d, smem);
 }
 
 // Rows per lane and most waves of a workgroup: the state of a pixel is 5 (TV)
@@ -412,7 +418,14 @@ void run_block(const Launch& L, const SliceDev& d, int kind, int dtype, bool fp1
     using B = decltype(cfg);
     constexpr bool TGV = decltype(tgv)::value;
     const size_t lds = size_t(2 * s.waves + 1) * (TGV ? 3 : 1) * 64 * sizeof(P);
-    hipLaunchKernelGGL((k_den_block<P, S, TGV, B::J, 64 * B::NW>), dim3(s.grid), dim3(64 * s.waves), lds, L.stream, a);
+    auto launch = [&](auto any) {
+      hipLaunchKernelGGL((k_den_block<P, S, TGV, B::J, 64 * B::NW, decltype(any)::value>), dim3(s.grid), dim3(64 * s.waves), lds,
+                         L.stream, a);
+    };
+    if constexpr (TGV && sizeof(typename RealOf<P>::T) == 4) {
+      if (std::min(d.alpha0, d.alpha1) < kTinyRadius) return launch(std::integral_constant<bool, true>{});
+    }
+    launch(std::integral_constant<bool, false>{});
   });
 }
 

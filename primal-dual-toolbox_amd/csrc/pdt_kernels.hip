@@ -692,7 +692,7 @@ __device__ __forceinline__ R sched_alpha(const SliceDev& d, double a_start, doub
 // pixel's values in memory).
 template <class P, class S, bool TGV, bool GAP>
 __device__ __forceinline__ void dual_pixel(const SliceDev& d, int x, int y, typename RealOf<P>::T sigma,
-                                           typename RealOf<P>::T w0, typename RealOf<P>::T w1,
+                                           Ball<typename RealOf<P>::T> w0, Ball<typename RealOf<P>::T> w1,
                                            double* t) {
   using L = Ld<P, S>;
   const int W = d.W, H = d.H;
@@ -787,7 +787,7 @@ __global__ __launch_bounds__(NT) void k_tv_dual(const SliceDev* sl, const int2* 
   for (int idx = threadIdx.x; idx < cnt; idx += NT) {
     const int yy = idx / W;
     const int x = idx - yy * W, y = ya + yy;
-    dual_pixel<P, P, false, GAP>(d, x, y, sigma, R(0), ball_weight(R(1)), t);
+    dual_pixel<P, P, false, GAP>(d, x, y, sigma, ball_any(R(1)), ball_any(R(1)), t);
     if (GAP) {
       const size_t i = size_t(y) * W + x;
       t[3] += dabs2(ub[i] - f[i]);
@@ -880,7 +880,8 @@ __global__ __launch_bounds__(NT) void k_tgv_dual(const SliceDev* sl, const int2*
   using R = typename RealOf<P>::T;
   const int W = d.W, H = d.H;
   const int ya = it.y, yb = min(H, ya + rpi);
-  const R sigma = R(d.sigma), w0 = ball_weight(R(d.alpha0)), w1 = ball_weight(R(d.alpha1));
+  const R sigma = R(d.sigma);
+  const auto w0 = ball_any(R(d.alpha0)), w1 = ball_any(R(d.alpha1));
   const auto ub = gptr<const P>(d.ub);
   const auto f = gptr<const P>(d.f);
   double t[kGapTerms] = {0};
@@ -918,7 +919,8 @@ __global__ __launch_bounds__(NT) void k_tgv_dual2(const SliceDev* sl, const int2
   const int W = d.W, H = d.H;
   const size_t n = size_t(W) * H;
   const int ya = it.y, yb = min(H, ya + rpi);
-  const R sigma = R(d.sigma), w0 = ball_weight(R(d.alpha0)), w1 = ball_weight(R(d.alpha1));
+  const R sigma = R(d.sigma);
+  const auto w0 = ball_any(R(d.alpha0)), w1 = ball_any(R(d.alpha1));
   const auto ub = gptr<const P>(d.ub);
   const auto ubp = gptr<const Pair<P>>(d.ub);
   const auto vbx = gptr<const P>(d.vb);
@@ -1112,8 +1114,8 @@ __device__ __forceinline__ void dual_workgroup(const SliceDev& d, int nd, double
   const int pa = min(WH, b * chunk), pe = min(WH, pa + chunk);
   const int k = gptr<int>(d.ctl)[CTL_ITER];
   const R sigma = R(d.sigma);
-  const R w0 = ball_weight(sched_alpha<R>(d, d.alpha0, d.alpha0_end, k));
-  const R w1 = ball_weight(sched_alpha<R>(d, d.alpha1, d.alpha1_end, k));
+  const auto w0 = ball_any(sched_alpha<R>(d, d.alpha0, d.alpha0_end, k));
+  const auto w1 = ball_any(sched_alpha<R>(d, d.alpha1, d.alpha1_end, k));
   const float rW = 1.0f / float(W);
   // GAP: the sums are formed as by 256 threads whatever NT is (wave w takes
   // the pixels of waves w, w + NT / 64, ... of those), so that every launch
@@ -1225,7 +1227,7 @@ __device__ __forceinline__ void rows_fwd(const SliceDev* sl, const int2* items, 
     const R sigma = R(d.sigma);
     const R a0 = sched_alpha<R>(d, d.alpha0, d.alpha0_end, k);
     const R a1 = sched_alpha<R>(d, d.alpha1, d.alpha1_end, k);
-    const R w0 = ball_weight(a0), w1 = ball_weight(a1);
+    const auto w0 = ball_any(a0), w1 = ball_any(a1);
     for (int x = xa + threadIdx.x; x < xe; x += NT) dual_pixel<C, C, MODE == M_TGV, GAP>(d, x, y, sigma, w0, w1, t);
   }
   if (NF > 0) {

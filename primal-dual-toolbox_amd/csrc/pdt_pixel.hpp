@@ -152,18 +152,41 @@ __device__ __forceinline__ double ball_weight(double alpha) { return rcp(alpha);
 __device__ __forceinline__ float ball_scale(float s, float w) { return fminf(1.f, w * __builtin_amdgcn_rsqf(s)); }
 __device__ __forceinline__ double ball_scale(double s, double w) { return rcp(fmax(1.0, sqrt(s) * w)); }
 
+// The same for any radius: the hardware takes a subnormal s (|b| < 2^-63) for
+// zero, hence for inside of every ball, so radii below 2^-63 scale s by 2^24
+// first, which makes every s normal (and takes |b| above 2^52 for infinite,
+// whose projection is zero).  The product by 1 of the other radii changes no
+// bit; it costs the blocked TGV launches 4 % (512 x 512 complex, 1000
+// iterations 3.59 against 3.45 ms), which take it for those radii only, and
+// the MRI dual steps nothing (320 x 320, 15 coils, 300 iterations 8.36 ms
+// against 8.37).
+constexpr double kTinyRadius = 0x1p-63;
+template <class R> struct Ball {
+  R w;
+};
+template <> struct Ball<float> {
+  float w, s;  // weight, scale of |b|^2
+};
+__device__ __forceinline__ Ball<double> ball_any(double alpha) { return {ball_weight(alpha)}; }
+__device__ __forceinline__ Ball<float> ball_any(float alpha) {
+  const bool tiny = alpha < float(kTinyRadius);
+  return {ball_weight(alpha) * (tiny ? 0x1p12f : 1.f), tiny ? 0x1p24f : 1.f};
+}
+__device__ __forceinline__ double ball_scale(double s, Ball<double> b) { return ball_scale(s, b.w); }
+__device__ __forceinline__ float ball_scale(float s, Ball<float> b) { return ball_scale(s * b.s, b.w); }
+
 // The arithmetic of the dual step at one pixel, on values: c = ubar, uxp /
 // uyp = ubar at the forward neighbours (c itself at the last column / row);
 // TGV: vx0, vy0 = vbar, vxx = vbar_x and vyx = vbar_y at the x neighbour,
 // vxy, vyy at the y neighbour.  Updates p (and q) in place, with optional
 // gap terms t[0] += |grad ub - vb|, t[1] += |E vb|_F, t[2] += Re<grad ub -
 // vb, p> + Re<E vb, q>_F (TGV_dual_p_kernel / TGV_dual_q_kernel /
-// TV_dual_p_kernel).  w0, w1: ball_weight of alpha0 (q; TGV only) and alpha1
-// (p; 1 for TV).
-template <class P, bool TGV, bool GAP>
+// TV_dual_p_kernel).  w0, w1: ball_weight or ball_any of alpha0 (q; TGV only)
+// and alpha1 (p; 1 for TV).
+template <class P, bool TGV, bool GAP, class B>
 __device__ __forceinline__ void dual_math(P c, P uxp, P uyp, P vx0, P vy0, P vxx, P vyx, P vxy, P vyy, P& px, P& py,
-                                          P& qxx, P& qyy, P& qxy, typename RealOf<P>::T sigma,
-                                          typename RealOf<P>::T w0, typename RealOf<P>::T w1, double* t) {
+                                          P& qxx, P& qyy, P& qxy, typename RealOf<P>::T sigma, B w0, B w1,
+                                          double* t) {
   using R = typename RealOf<P>::T;
   P tx = uxp - c, ty = uyp - c;
   if (TGV) {

@@ -145,9 +145,11 @@ template <> __device__ __forceinline__ float rcp<float>(float x) { return __buil
 // times the hardware's reciprocal square root (within 1 ulp), a rounding less
 // than sqrt, a product with 1 / alpha and a reciprocal, and 15 instructions
 // fewer (the correctly rounded sqrt alone takes about 12).  Double precision:
-// correctly rounded steps.  s = 0 gives 1; a negative or NaN alpha projects
-// nothing.
-__device__ __forceinline__ float ball_weight(float alpha) { return alpha >= 0.f ? alpha : __builtin_inff(); }
+// correctly rounded steps.  s = 0 gives 1; a negative (-0 too, as max(1, |b| /
+// alpha) has it) or NaN alpha projects nothing.
+__device__ __forceinline__ float ball_weight(float alpha) {
+  return alpha >= 0.f && !__builtin_signbit(alpha) ? alpha : __builtin_inff();
+}
 __device__ __forceinline__ double ball_weight(double alpha) { return rcp(alpha); }
 __device__ __forceinline__ float ball_scale(float s, float w) { return fminf(1.f, w * __builtin_amdgcn_rsqf(s)); }
 __device__ __forceinline__ double ball_scale(double s, double w) { return rcp(fmax(1.0, sqrt(s) * w)); }

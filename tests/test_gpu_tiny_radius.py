@@ -58,3 +58,21 @@ def test_reconstruction_at_a_tiny_radius(oracle, n, n_pe, coils):
     free = oracle.solve(oracle.TGV_MRI, k.astype(np.complex128), alpha0=1.0, alpha1=1.0, **prm)[0]
     assert rel_l2(free * 1e20, want * 1e20) > 10 * TOL
     assert rel_l2(o.getResult().astype(np.complex128) * 1e20, want * 1e20) < TOL
+
+
+@pytest.mark.parametrize("tile", [None, (52, 20, 6)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_negative_zero_projects_nothing(dtype, tile):
+    """max(1, |b| / alpha) is 1 for every alpha below zero, -0.0 among them."""
+    import primaldualtoolbox as pdt
+    f = np.random.default_rng(2).standard_normal((40, 50)).astype(dtype)
+    out = []
+    for radius in (-0.0, -1.0):
+        opt = pdt.denoising.TgvOptimizer_2f(dtype=dtype)
+        opt.setNoisyData(f)
+        p = opt.getParameters()
+        p.Lambda, p.alpha0, p.alpha1, p.max_iter = 5, radius, radius, 9
+        pdt.denoising.set_tiles([opt], rpi=1, tv_block=tile)
+        opt.solve()
+        out.append(opt.getResult().copy())
+    np.testing.assert_array_equal(*out)

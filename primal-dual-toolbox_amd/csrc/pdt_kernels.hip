@@ -28,6 +28,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <type_traits>
 
@@ -2693,8 +2694,14 @@ template <class R>
 static void op_forward(const Launch& L, const SliceDev& d) {
   constexpr int NR = kRowThreads;
   SliceDev* const dst = const_cast<SliceDev*>(L.sl);
-  // zeroing workgroups: 32 elements per thread
-  const int nz = int((int64_t(d.W) * d.Hk * d.C + 32 * NR - 1) / (32 * NR));
+  // zeroing workgroups: 32 elements per thread.  An output that overlaps the
+  // input is zeroed before the row transforms read it, not beside them.
+  const size_t in = size_t(d.W) * d.H, out = size_t(d.W) * d.Hk * d.C;
+  const auto x = static_cast<const Cx<R>*>(d.op_in);
+  const auto y = static_cast<const Cx<R>*>(d.op_out);
+  const bool overlap = std::less<>()(x, y + out) && std::less<>()(y, x + in);
+  if (overlap) run_zero(L.stream, d.op_out, out * sizeof(Cx<R>));
+  const int nz = overlap ? 0 : int((out + 32 * NR - 1) / (32 * NR));
   with_fft_len<R>(L.fft_w, [&](auto nf) {
     PDT_LAUNCH_NT((k_op_rows_fwd<R, NR, decltype(nf)::value>), L.nrg + nz, NR, L.lds_rows, L.stream, d, dst, L.nrg, L.cb, nz);
   });

@@ -20,13 +20,13 @@
 #include <random>
 #include <sstream>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "pdt_capi.h"
 #include "pdt_cnn.hpp"
 #include "pdt_desc.hpp"
 #include "pdt_launch.hpp"
+#include "pdt_pool.hpp"
 #include "pdt_tune.hpp"
 
 using namespace pdt;
@@ -1614,10 +1614,7 @@ void solve_pool(const std::vector<pdt_solver*>& sv, int streams, F&& solve_one) 
       }
     }
   };
-  std::vector<std::thread> pool;
-  for (int t = 1; t < std::min(streams, count); ++t) pool.emplace_back(work);
-  work();
-  for (auto& t : pool) t.join();
+  run_workers(std::min(streams, count), work);
   if (err_code != PDT_OK) fail(err_code, err_msg);
 }
 

@@ -94,7 +94,10 @@ typedef struct pdt_stats {
   double dual;        /* last dual value D                                     */
   double gap;         /* P - D                                                 */
   double rel_gap;     /* (P - D) / |P|                                         */
-  double ms;          /* device time of the iteration loop (hipEvent), ms      */
+  double ms;          /* device time of the iteration loop (hipEvent), ms; of a
+                         batched solve, the loop of all its slices (concurrent
+                         single solves: from the start of the first one's loop to
+                         the end of the last one's)                            */
   int32_t converged;  /* 1 if gap_tol was reached                              */
   double ms_to_stop;  /* NEW: in a batched solve, host time from the start of the
                          loop to the end of the chunk in which this slice stopped;

@@ -769,6 +769,36 @@ TuneKey mri_key(const std::vector<pdt_solver*>& sv) {
 // ---------------------------------------------------------------------------
 // The engine: one or many slices, persistent work lists, graph-replayed chunks
 // ---------------------------------------------------------------------------
+// A solve's iteration loop: its start and end on the device, its start and the
+// end of the chunk in which the (last) slice stopped on the host.
+struct LoopTimes {
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  std::chrono::steady_clock::time_point begin, stop;
+  LoopTimes() = default;
+  ~LoopTimes() {
+    for (hipEvent_t e : {e0, e1})
+      if (e) (void)hipEventDestroy(e);
+  }
+  LoopTimes(const LoopTimes&) = delete;
+  LoopTimes& operator=(const LoopTimes&) = delete;
+  void start(hipStream_t st) {
+    for (hipEvent_t* e : {&e0, &e1})
+      if (!*e) HIPC(hipEventCreate(e));
+    HIPC(hipEventRecord(e0, st));
+    begin = stop = std::chrono::steady_clock::now();
+  }
+  void end(hipStream_t st) {
+    HIPC(hipEventRecord(e1, st));
+    HIPC(hipEventSynchronize(e1));
+  }
+  // from the start of `first` to the end of this loop
+  float since(const LoopTimes& first) const {
+    float ms = 0;
+    HIPC(hipEventElapsedTime(&ms, first.e0, e1));
+    return ms;
+  }
+};
+
 struct Engine {
   int kind = 0, dtype = 0;
   bool fp16 = false;
@@ -811,6 +841,7 @@ struct Engine {
     hipGraphExec_t exec;
   };
   std::vector<GraphEntry> graphs;
+  LoopTimes loop;  // of the last run
 
   ~Engine() {
     SetupLock lk(g_setup_mu);
@@ -1397,10 +1428,7 @@ struct Engine {
     const bool use_graph = sv[0]->prm.use_graph != 0;
     std::vector<double> stop_ms(ns, -1.0);  // batched solves: time from the start to each slice's stop
     reset_ctl();
-    hipEvent_t e0, e1;
-    HIPC(hipEventCreate(&e0));
-    HIPC(hipEventCreate(&e1));
-    HIPC(hipEventRecord(e0, stream));
+    loop.start(stream);
     auto boundary = [&](unsigned k) {
       unsigned b = std::min(total, (k / chunk + 1) * chunk);
       if (gap) b = std::min(b, (k / gap_every + 1) * gap_every);
@@ -1458,6 +1486,7 @@ struct Engine {
         --nq;
         HIPC(hipEventSynchronize(ev_q[q]));
         std::memcpy(h_cs, h_cs_q[q], cs_bytes);
+        if (live) loop.stop = std::chrono::steady_clock::now();
         report();
         if (h_ctl[CTL_NGAP] > seen_ngap) {
           seen_ngap = h_ctl[CTL_NGAP];
@@ -1468,7 +1497,6 @@ struct Engine {
       }
     } else {
       unsigned k = 0;
-      const auto t0 = std::chrono::steady_clock::now();
       while (k < total) {
         const unsigned b = boundary(k);
         launch_chunk(int(b - k), gap && (b % gap_every) == 0, use_graph, k == 0);
@@ -1477,7 +1505,7 @@ struct Engine {
         k = b;
         // the end of the chunk in which a slice stopped (at its gap, seen in
         // the copied control words, or at its limit, below) is its time to stop
-        const double el = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        const double el = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - loop.begin).count();
         for (int i = 0; i < ns; ++i)
           if (stop_ms[i] < 0 && (!h_ctl[size_t(i) * CTL_WORDS + CTL_ACTIVE] || limit[i] <= k)) stop_ms[i] = el;
         // a slice stops at its own iteration limit (host-driven, so that no
@@ -1499,12 +1527,8 @@ struct Engine {
         compact_lists();
       }
     }
-    HIPC(hipEventRecord(e1, stream));
-    HIPC(hipEventSynchronize(e1));
-    float ms = 0;
-    HIPC(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    loop.end(stream);
+    const float ms = loop.since(loop);
     for (int i = 0; i < ns; ++i) {
       pdt_solver* s = sv[i];
       const int* c = h_ctl + size_t(i) * CTL_WORDS;
@@ -1582,9 +1606,9 @@ void check_batch(const std::vector<pdt_solver*>& sv) {
   }
 }
 
-// Runs solve_one on every solver, `streams` at a time: the calling thread and
-// streams - 1 more take the next solver in order; the first failure stops the
-// others from taking more and is thrown here.
+// Runs solve_one on the index of every solver, `streams` at a time: the
+// calling thread and streams - 1 more take the next solver in order; the first
+// failure stops the others from taking more and is thrown here.
 template <class F>
 void solve_pool(const std::vector<pdt_solver*>& sv, int streams, F&& solve_one) {
   const int count = (int)sv.size();
@@ -1602,7 +1626,7 @@ void solve_pool(const std::vector<pdt_solver*>& sv, int streams, F&& solve_one) 
         if (failed.load()) return;
         const int i = next.fetch_add(1);
         if (i >= count) return;
-        solve_one(sv[i]);
+        solve_one(i);
       }
     });
     if (rc != PDT_OK) {
@@ -1621,7 +1645,8 @@ void solve_pool(const std::vector<pdt_solver*>& sv, int streams, F&& solve_one) 
 // One prepared solver alone, on its cached engine: its work lists and
 // instantiated graphs stay valid while nothing they depend on changed (a
 // replaced engine is released, and the new one built, under the set-up lock).
-void solve_single(pdt_solver* s, int verbose) {
+// Returns the engine.
+std::shared_ptr<Engine> solve_single(pdt_solver* s, int verbose) {
   std::shared_ptr<Engine> cached;
   {
     SetupLock lk(g_setup_mu);
@@ -1641,6 +1666,7 @@ void solve_single(pdt_solver* s, int verbose) {
     }
   }
   cached->run(verbose);
+  return cached;
 }
 
 // Whether a batch of prepared operator solvers is faster as single solves on
@@ -1675,14 +1701,18 @@ void solve_many(std::vector<pdt_solver*>& sv, int verbose) {
     return;
   }
   if (batch_as_singles(sv, verbose)) {
-    const auto t0 = std::chrono::steady_clock::now();
-    auto since = [&] { return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count(); };
-    solve_pool(sv, kBatchStreams, [&](pdt_solver* s) {
-      solve_single(s, verbose);
-      s->stats.ms_to_stop = since();
-    });
-    const double ms = since();
-    for (auto* s : sv) s->stats.ms = ms;  // the loop's time, as of one set of launches
+    std::vector<std::shared_ptr<Engine>> es(sv.size());
+    solve_pool(sv, kBatchStreams, [&](int i) { es[i] = solve_single(sv[i], verbose); });
+    // the batch's loop is that of all solves: from the start of the first one
+    const LoopTimes* first = &es[0]->loop;
+    for (const auto& e : es)
+      if (e->loop.begin < first->begin) first = &e->loop;
+    float ms = 0;
+    for (const auto& e : es) ms = std::max(ms, e->loop.since(*first));
+    for (size_t i = 0; i < sv.size(); ++i) {
+      sv[i]->stats.ms = ms;
+      sv[i]->stats.ms_to_stop = std::chrono::duration<double, std::milli>(es[i]->loop.stop - first->begin).count();
+    }
     return;
   }
   auto e = std::make_unique<Engine>();
@@ -2513,8 +2543,8 @@ int pdt_solve_concurrent(pdt_solver** solvers, int count, int streams, int verbo
       for (int j = 0; j < i; ++j)
         if (v[j] == v[i]) fail(PDT_ERR_ARG, "a solver appears twice in the batch");
     }
-    solve_pool(v, streams, [&](pdt_solver* s) {
-      std::vector<pdt_solver*> one{s};
+    solve_pool(v, streams, [&](int i) {
+      std::vector<pdt_solver*> one{v[i]};
       solve_many(one, verbose);
     });
   });

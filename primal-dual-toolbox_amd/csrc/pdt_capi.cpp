@@ -57,6 +57,7 @@ struct Err {
 
 void hip_check(hipError_t e, const char* what) {
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // thrown here, not found again by the next call's check
     std::ostringstream ss;
     ss << what << ": " << hipGetErrorString(e);
     fail(PDT_ERR_HIP, ss.str());
@@ -2563,7 +2564,6 @@ struct pdt_cnn {
   DevBuf w, g, m, v;           // fp32 parameters, gradient, Adam moments
   std::vector<DevBuf> wk, wt;  // packed bf16 weights (forward, backward-data)
   int64_t step = 0;
-  int64_t cap = 0;             // pixels the activation buffers hold
   DevBuf y, dza, dzb, part, lpart;
   std::vector<DevBuf> act;     // hidden activations (bf16), nl - 1 of them
   DevBuf ws_x, ws_u, ws_v, ws_ss;  // warm-start input, (u0, v0) and sum of |A^*f|^2
@@ -2579,10 +2579,10 @@ struct pdt_cnn {
   const float* W(int l) const { return w.as<float>() + off[l]; }
   const float* b(int l) const { return w.as<float>() + off[l] + wsize(l); }
 
+  // activation buffers for P pixels (each knows its own size, so an allocation
+  // that fails leaves none of them shorter than it says)
   void ensure(int64_t P) {
-    if (P <= cap) return;
-    for (int l = 0; l + 1 < nl; ++l) act[l].alloc(size_t(P) * ch[l + 1] * 2);
-    cap = P;
+    for (int l = 0; l + 1 < nl; ++l) act[l].ensure(size_t(P) * ch[l + 1] * 2);
   }
 
   std::vector<CnnLayer> layers() const {

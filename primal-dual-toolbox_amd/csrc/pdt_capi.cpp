@@ -2173,8 +2173,8 @@ void profile_engine(std::vector<pdt_solver*> sv, int reps, pdt_kernel_prof* out,
       // temporally blocked launches, as a solve runs them: a graph of reps
       // pairs of launches timed with an event pair; per launch (tb_k
       // iterations) each plane read or written once: ROF reads u, ubar, p,
-      // f and writes u, ubar, p; TGV reads u, v, p, q, f and writes u, ubar,
-      // v, vbar, p, q
+      // f and writes u, ubar, p; TGV reads u, v, p, q, f and writes u, v, p,
+      // q
       hipEvent_t e0, e1;
       HIPC(hipEventCreate(&e0));
       HIPC(hipEventCreate(&e1));
@@ -2204,7 +2204,7 @@ void profile_engine(std::vector<pdt_solver*> sv, int reps, pdt_kernel_prof* out,
       double bytes = 0;
       for (auto* s : sv) {
         const double N = double(s->W) * s->H, pe = double(s->pe()), pq = double(s->pq_e());
-        bytes += e.kind == PDT_SOLVER_TGV ? (10 * pe + 10 * pq) * N : (5 * pe + 4 * pq) * N;
+        bytes += e.kind == PDT_SOLVER_TGV ? (7 * pe + 10 * pq) * N : (5 * pe + 4 * pq) * N;
       }
       *n = 0;
       if (cap > 0) {

@@ -301,12 +301,20 @@ __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
   if (blockIdx.x == 0 && threadIdx.x == 0) gptr<int>(d.ctl)[CTL_ITER] += k;
 }
 
-template <class P, class S, bool TGV, int J, int NT, bool ANY>
-__global__ __launch_bounds__(NT) void k_den_block(BlockArgs d) {
+template <class P, class S, bool TGV, int J, bool ANY>
+__device__ __forceinline__ void den_block(const BlockArgs& d, char* smem) {
+  if (int(blockDim.x >> 6) * J > d.H) block_iterations<P, S, TGV, J, true, ANY>(d, reinterpret_cast<P*>(smem));
+  else block_iterations<P, S, TGV, J, false, ANY>(d, reinterpret_cast<P*>(smem));
+}
+template <class P, int J, int NT>
+__global__ __launch_bounds__(NT) void k_tv_block(BlockArgs d) {
   extern __shared__ char smem_raw[];
-  P* const smem = reinterpret_cast<P*>(smem_raw);
-  if (int(blockDim.x >> 6) * J > d.H) block_iterations<P, S, TGV, J, true, ANY>(d, smem);
-  else block_iterations<P, S, TGV, J, false, ANY>(d, smem);
+  den_block<P, P, false, J, false>(d, smem_raw);
+}
+template <class P, class S, int J, int NT, bool ANY>
+__global__ __launch_bounds__(NT) void k_tgv_block(BlockArgs d) {
+  extern __shared__ char smem_raw[];
+  den_block<P, S, true, J, ANY>(d, smem_raw);
 }
 
 // Rows per lane and most waves of a workgroup: the state of a pixel is 5 (TV)
@@ -418,14 +426,19 @@ void run_block(const Launch& L, const SliceDev& d, int kind, int dtype, bool fp1
     using B = decltype(cfg);
     constexpr bool TGV = decltype(tgv)::value;
     const size_t lds = size_t(2 * s.waves + 1) * (TGV ? 3 : 1) * 64 * sizeof(P);
-    auto launch = [&](auto any) {
-      hipLaunchKernelGGL((k_den_block<P, S, TGV, B::J, 64 * B::NW, decltype(any)::value>), dim3(s.grid), dim3(64 * s.waves), lds,
-                         L.stream, a);
-    };
-    if constexpr (TGV && sizeof(typename RealOf<P>::T) == 4) {
-      if (std::min(d.alpha0, d.alpha1) < kTinyRadius) return launch(std::integral_constant<bool, true>{});
+    constexpr int J = B::J, NT = 64 * B::NW;
+    const dim3 grid(s.grid), block(64 * s.waves);
+    if constexpr (!TGV) {
+      hipLaunchKernelGGL((k_tv_block<P, J, NT>), grid, block, lds, L.stream, a);
+    } else {
+      if constexpr (sizeof(typename RealOf<P>::T) == 4) {
+        if (std::min(d.alpha0, d.alpha1) < kTinyRadius) {
+          hipLaunchKernelGGL((k_tgv_block<P, S, J, NT, true>), grid, block, lds, L.stream, a);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((k_tgv_block<P, S, J, NT, false>), grid, block, lds, L.stream, a);
     }
-    launch(std::integral_constant<bool, false>{});
   });
 }
 

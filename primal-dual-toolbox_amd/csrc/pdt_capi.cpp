@@ -583,8 +583,9 @@ struct pdt_solver {
   std::unique_ptr<pdt_array> u, v;  // result handles (u: {W,H}, v: {W,H,2})
   DevBuf ub, vb, p, q, tmp;
   // second copy of the state for the temporally blocked denoising launches:
-  // u, ubar, p (ROF and TGV) and v, vbar, q (TGV)
-  DevBuf u2, ub2, p2, v2, vb2, q2;
+  // u, p and ubar (ROF) or v, q (TGV, whose ubar and vbar no launch reads from
+  // the one before)
+  DevBuf u2, ub2, p2, v2, q2;
   DevBuf fk, rk, T1, T2, wpart;
   // set-up buffers kept across solves: descriptor and item list of the data
   // compaction, its partial sums, A^*f, and two reduction results
@@ -657,12 +658,11 @@ void alloc_state(pdt_solver* s, int W, int H) {
   }
   if (s->kind == PDT_SOLVER_TV || s->kind == PDT_SOLVER_TGV) {
     exact(s->u2, n * e);
-    exact(s->ub2, n * e);
     exact(s->p2, 2 * n * s->pq_e());
   }
+  if (s->kind == PDT_SOLVER_TV) exact(s->ub2, n * e);
   if (s->kind == PDT_SOLVER_TGV) {
     exact(s->v2, 2 * n * e);
-    exact(s->vb2, 2 * n * e);
     exact(s->q2, 3 * n * s->pq_e());
   }
   s->W = W;
@@ -978,7 +978,6 @@ struct Engine {
       d.ub2 = s->ub2.p;
       d.p2 = s->p2.p;
       d.v2 = s->v2.p;
-      d.vb2 = s->vb2.p;
       d.q2 = s->q2.p;
       d.f = s->f->ptr;
       if (mri) {

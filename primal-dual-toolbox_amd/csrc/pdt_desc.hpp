@@ -79,13 +79,12 @@ struct SliceDev {
   const void* f;  // denoising data
   void* tmp;      // 2 planes: TGV dual-restoration scratch
   // the second copy of the state that the temporally blocked denoising
-  // launches write and read in turn (ping-pong): u, ubar, p (2 planes) and,
-  // for TGV, v, vbar (2 planes each) and q (3 planes)
+  // launches write and read in turn (ping-pong): u, p (2 planes) and, for ROF,
+  // ubar, for TGV v (2 planes) and q (3 planes)
   void* u2;
   void* ub2;
   void* p2;
   void* v2;
-  void* vb2;
   void* q2;
   // geometry
   int W, H;       // image {W (x, contiguous), H (y)}

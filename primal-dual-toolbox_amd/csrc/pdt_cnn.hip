@@ -631,13 +631,15 @@ __device__ __forceinline__ bf8 grad_frag(const bf4* s, int p, int c0) {
 __host__ __device__ constexpr int grad_ch(int cout) { return cout == 32 ? 32 : 16; }
 
 // Adds the accumulators of the block's waves in wave order and writes the
-// block's partial, [tile][lane][i] then db[co]; sum is the block's LDS.
+// block's partial, [tile][lane][i] then db[co]; sum is the block's LDS.  (The
+// barrier is at the head of a loop whose last LDS store is at its end:
+// wg_barrier, whose wait does not depend on the loop being unrolled.)
 template <int NT, int CT>
 __device__ __forceinline__ void grad_partial(const f4 (&acc)[NT], const f4 (&db)[CT], float* sum, float* part) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   f4* s4 = reinterpret_cast<f4*>(sum);
   for (int q = 0; q < kGradWaves; ++q) {
-    __syncthreads();
+    wg_barrier();
     if (wave == q) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) s4[t * 64 + lane] = q ? s4[t * 64 + lane] + acc[t] : acc[t];
@@ -650,7 +652,7 @@ __device__ __forceinline__ void grad_partial(const f4 (&acc)[NT], const f4 (&db)
         }
     }
   }
-  __syncthreads();
+  wg_barrier();
   constexpr int N4 = NT * 64 + CT * 4;
   f4* o = reinterpret_cast<f4*>(part) + size_t(blockIdx.x) * N4;
   for (int e = threadIdx.x; e < N4; e += kGradThreads) o[e] = s4[e];

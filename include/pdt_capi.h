@@ -230,8 +230,9 @@ typedef struct pdt_tiles {
                       adjoint row and denoising passes                          */
   int32_t tb_x, tb_y, tb_k; /* ROF or TGV denoising, one slice: tb_k
                       iterations per launch on tiles of tb_x x tb_y pixels
-                      and a halo of tb_k, cut to the 64 columns and the rows
-                      (32 or 64) a workgroup holds
+                      and a halo of tb_k.  A workgroup holds 64 columns, to
+                      which every tile is widened or cut, and as many rows as
+                      the tile and its halo take, up to 32 or 64
                       (tb_k 0: one iteration per pair of launches)               */
   int32_t dual_px; /* TGV denoising: pixels per thread of the dual step, 1 or 2
                       (2 needs even widths; 0: the default, 2 where possible)   */

@@ -98,12 +98,14 @@ void run_stage(const Launch& L, int kind, int dtype, bool fp16, bool gap, int st
 // The first iteration of a solve starts from stages 0 and 1 instead of 0.
 void run_pair_stage(const Launch& L, int kind, int dtype, int which, bool gap);
 // The launch of k blocked ROF or TGV (kind) iterations on a W x H slice with
-// interior tiles of tx x ty pixels: the exact region of a workgroup (at most
-// 64 columns and the rows its waves hold; tiles are cut to fit), its waves and
-// the number of workgroups (0: the halo leaves no interior).
+// interior tiles of tx x ty pixels: the rows of a workgroup's exact region
+// (whole waves of rows around the tile and its halo, as many as it holds; its
+// columns are kBlockCols, tiles are widened or cut to fit), its waves, the
+// number of workgroups (0: the halo leaves no interior) and of those in a row.
 struct BlockShape {
-  int rx = 0, ry = 0, waves = 0, grid = 0;
+  int ry = 0, waves = 0, grid = 0, nbx = 0;
 };
+constexpr int kBlockCols = 64;  // columns of a region, one per lane
 BlockShape block_shape(int kind, int dtype, int W, int H, int tx, int ty, int k);
 // The tile (x, y, iterations) of a W x H slice without a tuned or forced one,
 // and the ranges it is chosen from (iterations per launch, waves per

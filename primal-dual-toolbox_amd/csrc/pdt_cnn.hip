@@ -56,13 +56,6 @@ __device__ __forceinline__ bf8 keep(bf8 v, uint32_t m) {
   return __builtin_bit_cast(bf8, x);
 }
 
-// Workgroups go round-robin over the 8 XCDs: consecutive ones (neighbouring
-// strips and rows, which share input rows) to one XCD and its L2.
-__device__ __forceinline__ int xcd_block(int b, int n) {
-  const int q = n >> 3, r = n & 7, x = b & 7, k = b >> 3;
-  return x * q + min(x, r) + k;
-}
-
 // Input channels as the kernels see them (the 6-channel gradient as 8), the
 // 32-wide k-steps and the 16-wide output-channel tiles of a convolution.
 __host__ __device__ constexpr int chan_in(int cin) { return cin == 6 ? 8 : cin; }
@@ -87,7 +80,8 @@ __device__ __forceinline__ uint32_t strip_rows(int n, int h, int w, int width) {
 template <int WAVES>
 __device__ __forceinline__ Share share_of(uint32_t rows) {
   const uint32_t nw = gridDim.x * WAVES, q = rows / nw, r = rows - q * nw;
-  const uint32_t id = uint32_t(xcd_block(blockIdx.x, gridDim.x)) * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // (neighbouring strips and rows, which share input rows, to one XCD and its L2)
+  const uint32_t id = uint32_t(xcd_item(blockIdx.x, gridDim.x)) * WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t a = id * q + min(id, r);
   return {a, a + q + (id < r ? 1u : 0u)};
 }
@@ -572,7 +566,7 @@ __global__ __launch_bounds__(64 * kNetLayers) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(16))) bf8 ring[(kNetLayers - 1) * 2 * kNetPix * 4];
   __shared__ uint32_t taps[3 * kNetPix + 1];
   const int halo = depth - 1, ow = kNetCols - 2 * halo, ns = (w + ow - 1) / ow, nc = (h + R - 1) / R;
-  const int id = xcd_block(blockIdx.x, gridDim.x), img = id / (ns * nc), r = id - img * ns * nc, cy = r / ns;
+  const int id = xcd_item(blockIdx.x, gridDim.x), img = id / (ns * nc), r = id - img * ns * nc, cy = r / ns;
   const int s0 = (r - cy * ns) * ow, s1 = min(w, s0 + ow), xr = s0 - halo;
   const int y0 = cy * R, y1 = min(h, y0 + R), ya = y0 - halo;
   const size_t base = size_t(img) * h;

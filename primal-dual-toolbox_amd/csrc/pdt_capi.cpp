@@ -1669,28 +1669,22 @@ std::shared_ptr<Engine> solve_single(pdt_solver* s, int verbose) {
   return cached;
 }
 
-// Whether a batch of prepared operator solvers is faster as single solves on
-// kBatchStreams streams than as one work-list launch per pass and group of
-// equal transform lengths.  A group's launches follow one another, each with
-// its own tail, and stream every slice through DRAM; single solves overlap,
-// run paired iterations and keep fewer slices in the caches, but pay a chunk's
-// start per slice.  Measured per 100 iterations (n slices in G groups, X
-// million sensitivities on the image windows): batched about 2.2 G + 0.1 n +
-// 1.5 X ms, single 0.65 n + 0.85 X ms, equal at n = 4 G + 1.2 X.  Eight slices
-// of 320 x 320, 15 coils: 21.0 against 15.5 ms, of 64 x 64, 8 coils: 3.6
-// against 7.5; eight mixed slices in four groups: 29.1 against 17.9.  A batch
-// whose tiles were tuned or set keeps the launches they were chosen for, as do
-// direct launches (no graphs) and verbose solves.
+// Whether a batch of prepared operator solvers runs as single solves on
+// kBatchStreams streams (batch_singles_faster).  A batch whose tiles were tuned
+// or set keeps the launches they were chosen for, as do direct launches (no
+// graphs) and verbose solves.
 constexpr int kBatchStreams = 4;
 bool batch_as_singles(const std::vector<pdt_solver*>& sv, int verbose) {
   if (!sv[0]->is_op() || verbose || sv[0]->prm.use_graph == 0 || tune_has(mri_key(sv))) return false;
-  std::map<std::pair<int, int>, int> groups;
-  double x = 0;
+  std::vector<BatchSlice> b;
   for (auto* s : sv) {
-    groups[{s->op->W, s->op->Hk}]++;
-    x += 1e-6 * double(s->op->C) * s->W * s->H;
+    const pdt_op& o = *s->op;
+    // (rows of 368 pair too, but their radix-23 stages leave little to gain)
+    const bool paired = s->dtype == PDT_C64 && o.kind != PDT_OP_SAMPLING && o.W % 64 == 0 &&
+                        rows_adj_fused_ok(DT_C64, o.W, o.C, o.ncols);
+    b.push_back({o.W, o.Hk, 0.5e-6 * (is_dbl(s->dtype) ? 4 : 1) * o.C * double(o.W) * o.Hk, paired});
   }
-  return double(sv.size()) < 4.0 * double(groups.size()) + 1.2 * x;
+  return batch_singles_faster(b.data(), int(b.size()));
 }
 
 void solve_many(std::vector<pdt_solver*>& sv, int verbose) {

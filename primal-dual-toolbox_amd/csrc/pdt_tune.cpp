@@ -6,8 +6,10 @@
 #include <fstream>
 #include <map>
 #include <mutex>
+#include <set>
 #include <sstream>
 #include <tuple>
+#include <utility>
 
 namespace pdt {
 
@@ -92,6 +94,16 @@ void tune_store(const TuneKey& k, const TuneVal& v) {
   load_locked();
   g_cache[k] = v;
   save_locked();
+}
+
+bool batch_singles_faster(const BatchSlice* s, int n) {
+  std::set<std::pair<int, int>> groups;
+  double paired = 0, other = 0;
+  for (int i = 0; i < n; ++i) {
+    groups.insert({s[i].W, s[i].Hk});
+    (s[i].paired ? paired : other) += s[i].x;
+  }
+  return n + 1.5 < 3.5 * double(groups.size()) + 1.8 * paired + 0.4 * other;
 }
 
 }  // namespace pdt

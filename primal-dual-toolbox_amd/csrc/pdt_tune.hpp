@@ -34,4 +34,28 @@ TuneVal tune_lookup(const TuneKey& k);
 bool tune_has(const TuneKey& k);
 void tune_store(const TuneKey& k, const TuneVal& v);
 
+// A slice of a batch of operator solvers: its transform lengths, million
+// sensitivities on half the k-space grid (C W Hk / 2; 4 times in double
+// precision, whose passes take that much longer per element) and whether it
+// would run paired iterations alone.
+struct BatchSlice {
+  int W, Hk;
+  double x;
+  bool paired;
+};
+// Whether n slices are faster as single solves on a few streams than as one
+// work-list launch per pass and group of equal transform lengths.  A group's
+// launches follow one another, each with its own tail, and stream every slice
+// through DRAM; single solves overlap, pair their iterations where they can and
+// keep fewer slices in the caches, but pay every chunk's start per slice, and
+// three or more of them take 4 ms per 100 iterations however small they are.
+// Fitted to 378 batches of 2 to 32 slices (48 x 48 to 384 x 384, 1 to 15 coils,
+// up to four sizes, all three operators, both precisions), both ways measured
+// over 100 iterations: the way it takes is within 1 % of the faster one in the
+// mean and 11 % at the worst, and at the worst 4 % slower than the work lists.
+// On either side of the line: 8 slices of 320 x 320, 15 coils 21.3 ms batched
+// and 14.7 as singles; 2 of 48 x 48 and 64 x 64, 6 coils 5.3 and 2.2; 8 of 64 x
+// 64, 15 coils 4.4 and 7.5; 3 of 128 x 128, 4 coils 2.7 and 3.9.
+bool batch_singles_faster(const BatchSlice* s, int n);
+
 }  // namespace pdt

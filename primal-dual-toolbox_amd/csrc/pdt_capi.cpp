@@ -430,7 +430,7 @@ struct pdt_op {
     if (lds_cols_bytes(dt, 1, Hk) > init_kernel_attrs() || lds_rows_bytes(dt, 1, W, ncols) > init_kernel_attrs())
       fail(PDT_ERR_UNSUPPORTED, prefix() + "transform length too large for the LDS passes");
     cb_out = std::min(kDefaultCb, max_cb(dt, W, ncols, C));
-    cg_out = std::min(default_cg(Hk), max_cg(dt, Hk, ncols));
+    cg_out = std::min(default_cg(dt, Hk), max_cg(dt, Hk, ncols));
     lr = lds_rows_bytes(dt, cb_out, W, ncols);
     lc = lds_cols_bytes(dt, cg_out, Hk);
   }
@@ -882,7 +882,7 @@ struct Engine {
       int cg_max = maxNc, cg_def = maxNc;  // of every slice's column length
       for (auto* s : sv) {
         cg_max = std::min(cg_max, max_cg(dt, s->op->Hk, maxNc));
-        cg_def = std::min(cg_def, default_cg(s->op->Hk));
+        cg_def = std::min(cg_def, default_cg(dt, s->op->Hk));
       }
       key = mri_key(sv);
       TuneVal tv = tune_lookup(key);

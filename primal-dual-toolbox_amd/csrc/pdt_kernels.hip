@@ -1451,7 +1451,7 @@ __global__ __launch_bounds__(NT) void k_op_cols_adj(const SliceDev d, SliceDev* 
   cols<R, CM_ADJ, false, NT, NF, false, 0>(&d, nullptr, nitems, cg, nullptr, 0, nullptr, smem_raw);
 }
 
-// Column pass of the lengths 8 M 8 (with_direct_cols): a thread does one
+// Column pass of the lengths 8 M 8 (those of with_direct_cols): a thread does one
 // butterfly of every stage, and what comes before the first stage, between the
 // two transforms and after the last one stays in its registers.  The first
 // stage reads T1; the last stage of the forward transform leaves outputs
@@ -2469,6 +2469,7 @@ static void with_fft_len(int n, Fn&& fn) {
 template <class R, class Fn>
 static void with_other_len(int n, Fn&& fn) {
   if constexpr (std::is_same<R, float>::value) {
+    if (n == 256) return fn(std::integral_constant<int, 256>{});
     if (n == 368) return fn(std::integral_constant<int, 368>{});
     if (n == 736) return fn(std::integral_constant<int, 736>{});
   }
@@ -2476,10 +2477,21 @@ static void with_other_len(int n, Fn&& fn) {
 }
 
 // Calls fn(std::integral_constant<int, N>) when columns of n have k_cols_direct.
-template <class Fn>
+// Not for 256 points in single precision, where the general kernel is the
+// faster one: it spreads two columns over 256 threads, which leaves each less to
+// do one after the other.  us per launch, general against direct: 8 coils, 256
+// columns wide 4.53 against 4.97; 20 coils with the dual step 6.91 against 7.38;
+// an iteration of 256 x 256, 8 coils 12.5 against 13.0, 20 coils 17.4 against
+// 18.2.  In double precision (no other compile-time plan) direct is the faster.
+template <class R, class Fn>
 static bool with_direct_cols(int n, Fn&& fn) {
+  if constexpr (!std::is_same<R, float>::value) {
+    if (n == 256) {
+      fn(std::integral_constant<int, 256>{});
+      return true;
+    }
+  }
   switch (n) {
-    case 256: fn(std::integral_constant<int, 256>{}); return true;
     case 320: fn(std::integral_constant<int, 320>{}); return true;
     case 384: fn(std::integral_constant<int, 384>{}); return true;
     case 512: fn(std::integral_constant<int, 512>{}); return true;
@@ -2545,19 +2557,23 @@ static void launch_rows_adj(const Launch& L, bool gap) {
   }
 }
 
+// Columns that a group of k_cols_direct holds at most; 0: not its length.
+static int direct_cols(int dtype, int Hk) {
+  int cs = 0;
+  if (dtype == DT_C64) with_direct_cols<float>(Hk, [&](auto nf) { cs = ColShape<float, decltype(nf)::value>::CS; });
+  else with_direct_cols<double>(Hk, [&](auto nf) { cs = ColShape<double, decltype(nf)::value>::CS; });
+  return cs;
+}
+
 int max_cg(int dtype, int Hk, int nc) {
   int cg = nc > 1 ? nc : 1;
-  with_direct_cols(Hk, [&](auto nf) {
-    constexpr int CS = ColShape<float, decltype(nf)::value>::CS;
-    cg = cg < CS ? cg : CS;
-  });
+  if (const int cs = direct_cols(dtype, Hk)) cg = std::min(cg, cs);
   while (cg > 1 && lds_cols_bytes(dtype, cg, Hk) > init_kernel_attrs()) --cg;
   return cg;
 }
-int default_cg(int Hk) {
-  int cg = 2;
-  with_direct_cols(Hk, [&](auto nf) { cg = ColShape<float, decltype(nf)::value>::CS; });
-  return cg;
+int default_cg(int dtype, int Hk) {
+  const int cs = direct_cols(dtype, Hk);
+  return cs ? cs : 2;
 }
 
 // Column pass (DUAL: with the dual step's workgroups, gap terms to pd).
@@ -2566,7 +2582,7 @@ static void launch_cols(const Launch& L, const int2* items, int ndual, double* p
   constexpr int NC = kColThreads;
   const size_t limit = init_kernel_attrs();
   bool done = false;
-  with_direct_cols(L.fft_h, [&](auto nf) {
+  with_direct_cols<R>(L.fft_h, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     using Sh = ColShape<R, NF>;
     if (Sh::lds > limit) return;  // (a runtime that refuses more than 64 KB)
@@ -2712,7 +2728,7 @@ template <class R>
 static void op_adjoint(const Launch& L, const SliceDev& d) {
   SliceDev* const dst = const_cast<SliceDev*>(L.sl);
   bool done = false;
-  with_direct_cols(L.fft_h, [&](auto nf) {
+  with_direct_cols<R>(L.fft_h, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     using Sh = ColShape<R, NF>;
     if (Sh::lds > init_kernel_attrs()) return;
@@ -2807,8 +2823,8 @@ static bool set_lds_attrs(int b) {
     }
   };
   for (int n : kFftLengths) {
-    with_direct_cols(n, direct);
-    with_other_len<R>(n, col);  // (0 for the lengths of the line above)
+    with_direct_cols<R>(n, direct);
+    with_other_len<R>(n, col);  // (0 for other lengths)
   }
   with_fft_len<R>(0, one);
   for (int n : kFftLengths)

@@ -163,6 +163,6 @@ size_t lds_cols_bytes(int dtype, int cg, int Hk);
 // Columns per column group: the most a launch takes, and the number without a
 // tuned or forced choice.
 int max_cg(int dtype, int Hk, int nc);
-int default_cg(int Hk);
+int default_cg(int dtype, int Hk);
 
 }  // namespace pdt

@@ -206,14 +206,6 @@ int max_cb(int dt, int W, int nc, int C) {
   while (cb > 1 && lds_rows_bytes(dt, cb, W, nc) > init_kernel_attrs()) --cb;
   return cb;
 }
-// Default tiles before any autotuning: coils per row item (columns per column
-// group: default_cg; temporally blocked denoising: block_choose).  Single
-// slices on rows without a compile-time plan take 2, in single precision and
-// wherever all_coils holds: 350 x 400, 16 coils 81 us per iteration against 88
-// with 4; in double 256 x 256, 8 coils 27.0 against 27.8, but 320 x 320, 15
-// coils 74 against 73.
-constexpr int kDefaultCb = 4, kDefaultCbPlain = 2;
-
 // Whether a single slice's adjoint row pass holds every coil of a row in one
 // workgroup by default (no coil sums through memory, no k_mri_primal): where
 // the straight-line path fits, which also makes paired iterations (256 x 256,
@@ -889,8 +881,7 @@ struct Engine {
       for (int i = 0; i < 4; ++i) L.wpc[i] = force_wpc[i] >= 0 ? force_wpc[i] : tv.wpc[i];
       unpaired = force_unpaired >= 0 ? force_unpaired != 0 : tv.unpaired != 0;
       const bool one_group = ns == 1 && sv[0]->op->kind != PDT_OP_SAMPLING && all_coils(dt, maxW, maxC, maxNc);
-      const bool plain = ns == 1 && !fft_len_compiled(dt, maxW) && (one_group || dt == DT_C64);
-      const int cb_def = plain ? kDefaultCbPlain : kDefaultCb;
+      const int cb_def = ns == 1 ? default_cb(dt, maxW, sv[0]->H, maxC, maxNc, one_group) : kDefaultCb;
       cb = force_cb > 0 ? force_cb : force_cb < 0 ? cb_def : tv.cb > 0 ? tv.cb : cb_def;
       cg = force_cg > 0 ? force_cg : force_cg < 0 ? cg_def : tv.cg > 0 ? tv.cg : cg_def;
       const int def_cb_a = one_group ? maxC : cb;

@@ -2557,6 +2557,32 @@ static void launch_rows_adj(const Launch& L, bool gap) {
   }
 }
 
+// Two on rows without a compile-time plan, in single precision and wherever
+// one_group holds (double, 320 x 320, 15 coils, not one_group 74 us per iteration
+// against 73 with four), while the items of two and the dual step's workgroups
+// fit the chip's 2048 places for workgroups of 256 threads: up to about 1800
+// items (1200 in double precision, whose registers leave fewer places).  Above,
+// four are faster: us per iteration with two and four, 128 x 230, 20 coils (1280
+// items of two) 36.2 and 37.9; 320 x 64, 12 coils (1920) 20.8 and 18.5; 320 x 200,
+// 20 coils (3200) 35.7 and 32.7.  Where cb is the adjoint row pass's number too
+// (not one_group), fours must fit by their LDS as well: 256 x 300, 20 coils 44.2
+// and 36.8, 256 x 500, 16 coils (1024 items of four, 1024 places) 51.7 and 49.0,
+// 225 x 500, 20 coils (1125) 63.6 and 72.8; with six or more per CU they need
+// not, 400 x 270, 20 coils 1.08 times faster.  Measured at 982 sizes from 64 x 48
+// to 400 x 700; the rule's choice is at the worst 11 % off the better one, 0.3 %
+// in the mean.
+int default_cb(int dtype, int W, int H, int C, int nc, bool one_group) {
+  if (fft_len_compiled(dtype, W)) return kDefaultCb;
+  const long twos = long(H) * ((C + 1) / 2), fours = long(H) * ((C + 3) / 4);
+  if (dtype == DT_C128) return one_group && twos <= 1200 ? 2 : kDefaultCb;
+  if (twos <= 1800) return 2;
+  if (one_group) return kDefaultCb;
+  constexpr size_t kGranule = 1280;  // LDS is given out in these units
+  const size_t lds = (lds_rows_bytes(dtype, kDefaultCb, W, nc) + kGranule - 1) / kGranule * kGranule;
+  const long per_cu = long(kLdsMax / lds);
+  return per_cu >= 6 || fours <= 256 * per_cu ? kDefaultCb : 2;
+}
+
 // Columns that a group of k_cols_direct holds at most; 0: not its length.
 static int direct_cols(int dtype, int Hk) {
   int cs = 0;

@@ -160,6 +160,11 @@ size_t init_kernel_attrs();
 // row pass uses them unpadded)
 size_t lds_rows_bytes(int dtype, int cb, int W, int nc, bool padded = true);
 size_t lds_cols_bytes(int dtype, int cg, int Hk);
+// Default tiles before any autotuning.  Coils per row item: kDefaultCb, for a
+// single slice of H rows default_cb (one_group: its adjoint row pass holds every
+// coil in one item).
+constexpr int kDefaultCb = 4;
+int default_cb(int dtype, int W, int H, int C, int nc, bool one_group);
 // Columns per column group: the most a launch takes, and the number without a
 // tuned or forced choice.
 int max_cg(int dtype, int Hk, int nc);

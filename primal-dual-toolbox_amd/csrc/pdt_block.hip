@@ -75,6 +75,16 @@ struct BlockArgs {
   double tau, sigma, lambda, theta, alpha0, alpha1;
 };
 
+// A point of the program by which the memory accesses before it are issued and
+// the launch's parameters and output addresses are in registers.
+__device__ __forceinline__ void args_ready(const BlockArgs& d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" ::"s"(d.ou), "s"(d.ov), "s"(d.op), "s"(d.oq), "s"(d.tau), "s"(d.sigma), "s"(d.lambda), "s"(d.theta),
+               "s"(d.alpha0), "s"(d.alpha1)
+               : "memory");
+#endif
+}
+
 // k iterations (TV: TV_dual_p_kernel, TV_primal_u_kernel; TGV, primal step
 // first: TV_primal_u_kernel + TGV_primal_v_kernel, TGV_dual_p_kernel +
 // TGV_dual_q_kernel; tgv_kernels.cuh:225-324,568-605,647-686,
@@ -106,6 +116,12 @@ struct BlockArgs {
 // for bit.  TGV launches do not store ubar and vbar: the primal step, which
 // comes first, rewrites them.
 //
+// Bound by vector instructions and by what is left of the waits: a launch of 6
+// iterations of TGV on 512 x 512 complex pixels takes 19.6 us, of which the
+// vector instructions alone 10.4 (2.0 times the image's pixels, with the halo);
+// the waves wait 28 % of their time.  TGV with fp16 duals on 961 x 1100: 21.0
+// and 13.2 us, 33 %; 20 iterations of TV on 256 x 256: 13.2 and 9.2 us, 36 %.
+//
 // ANY: projection radii of any size (ball_any).
 template <class P, class S, bool TGV, int J, bool FLAT, bool ANY>
 __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
@@ -126,6 +142,8 @@ __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
   const size_t n = size_t(W) * H;
   P* const edge_dn = smem;                       // [NW + 1][NU][64], slot 0 zero
   P* const edge_up = smem + (NW + 1) * NU * 64;  // [NW][NU][64]
+  int active = 1;
+  if constexpr (TGV) active = gptr<const int>(d.ctl)[CTL_ACTIVE];
   P u[J], ub[J], f[J], px[J], py[J], vx[J], vy[J], vbx[J], vby[J], qxx[J], qyy[J], qxy[J];
   {
     const auto gu = gptr<const P>(d.u);
@@ -153,10 +171,21 @@ __device__ __forceinline__ void block_iterations(const BlockArgs& d, P* smem) {
     }
   }
   // A finished slice's workgroups leave before their first store.  The fence
-  // keeps the loads above ahead of this one's wait (the compiler moved them
-  // behind the branch: 14.0 us instead of 12.9 for 20 iterations of 256 x 256).
-  asm volatile("" ::: "memory");
-  if (gptr<const int>(d.ctl)[CTL_ACTIVE] == 0) return;
+  // keeps the loads above ahead of this one's wait, where the compiler moved
+  // them behind the branch.  ROF reads the control word after its few loads and
+  // waits for all of them at once (20 iterations of 256 x 256: 12.9 us, 13.8
+  // with the word first, 14.0 without the fence).  TGV reads it first, which
+  // keeps its 36 or more loads in flight until their values are stored to LDS,
+  // and has the launch's other arguments fetched here, not behind the branch one
+  // latency after the other (a launch on 474 x 1065 complex pixels 0.9 %, on 100
+  // x 120 1.2 %, on 256 x 300 in double 1.5 % shorter).
+  if constexpr (TGV) {
+    args_ready(d);
+  } else {
+    asm volatile("" ::: "memory");
+    active = gptr<const int>(d.ctl)[CTL_ACTIVE];
+  }
+  if (active == 0) return;
   if (wave == 0)
     for (int c = 0; c < NU; ++c) edge_dn[c * 64 + lane] = pzero<P>();
   auto put_dn = [&]() {
@@ -319,7 +348,8 @@ __global__ __launch_bounds__(NT) void k_tgv_block(BlockArgs d) {
 
 // Rows per lane and most waves of a workgroup: the state of a pixel is 5 (TV)
 // or 12 (TGV) values, in 512 / (waves per SIMD) registers.  Two rows per lane
-// measured the same, eight slower (they spill or halve the waves).
+// measured the same, eight slower (they spill or halve the waves).  Complex
+// double TGV spills 19 registers (80 bytes) with four.
 template <class P, bool TGV> struct BlockCfg;
 template <> struct BlockCfg<float, false> { static constexpr int J = kBlockRows, NW = 16; };
 template <> struct BlockCfg<Cx<float>, false> { static constexpr int J = kBlockRows, NW = 16; };
@@ -383,8 +413,10 @@ BlockShape block_shape(int kind, int dtype, int W, int H, int tx, int ty, int k)
 // CU at the row time of the type, whole waves on each of the 4 SIMDs.  More
 // iterations per launch share the first two out over more iterations and
 // widen the halo.  Fitted to 1900 measured (type, size, tile) times from 100
-// x 120 to 1000 x 1000; the tile it takes is within 2 % of the best of them
-// for 31 of the 40 types and sizes, 17 % at the worst.
+// x 120 to 1000 x 1000.  Against the best of 29 tiles, 10 types at 4 sizes: within
+// 2 % for 27 of the 40 and 5 % for 35; the worst are at 1000 x 1000, where fewer
+// rows per workgroup are faster (complex TGV 11.9 us per iteration and 9.7 with
+// 56 x 8 x 4, complex TV 4.28 and 3.62 with 48 x 32 x 8).
 void block_choose(int kind, int dtype, bool fp16, int W, int H, int tile[3]) {
   constexpr double kLaunchUs = 4.8, kBytesPerUs = 17e6;
   const bool tgv = kind == K_TGV;

@@ -213,9 +213,11 @@ typedef struct pdt_kernel_prof {
   double bytes;
 } pdt_kernel_prof;
 PDT_API int pdt_solver_profile(pdt_solver* s, int reps, pdt_kernel_prof* out, int cap, int* n);
-/* NEW: pdt_solver_profile over the launches of a batch (pdt_batch_solve):
- * per kernel, the duration of one launch over every slice and the
- * algorithmic bytes of that launch summed over the slices. */
+/* NEW: pdt_solver_profile over the work-list launches of a batch: per kernel,
+ * the duration of one launch over every slice and the algorithmic bytes of
+ * that launch summed over the slices.  Where pdt_batch_solve runs the batch as
+ * concurrent single solves, its launches are those pdt_solver_profile reports
+ * for each solver instead. */
 PDT_API int pdt_batch_profile(pdt_solver** solvers, int count, int reps, pdt_kernel_prof* out, int cap, int* n);
 
 /* NEW: tile shapes and launch shapes of the fused kernels, one choice per
@@ -258,7 +260,8 @@ PDT_API int pdt_autotune(pdt_solver** solvers, int count, int reps, pdt_tiles* o
 
 /* NEW: a manual tile choice for the shape of these solvers (one batch),
  * stored in the same tile cache as pdt_autotune's result: cb, cg, rpi, cb_a
- * <= 0 take the default (cb_a: every coil of a row in one adjoint workgroup
+ * <= 0 take the default (cb: 4, or 2 on rows without a compile-time plan while
+ * few enough items result; cb_a: every coil of a row in one adjoint workgroup
  * where a single slice's straight-line adjoint path fits, or, on rows without
  * a compile-time plan, two such workgroups fit a CU's LDS; else cb), values
  * above a shape's limit are clamped; wpc in
@@ -272,8 +275,9 @@ PDT_API int pdt_set_tiles(pdt_solver** solvers, int count, const pdt_tiles* tile
  * operator solvers of large slices or many sizes, as concurrent single solves
  * (pdt_solve_concurrent), whichever a rule on the sizes takes to be faster
  * (batches with tuned or set tiles, without graphs or verbose: always the
- * work lists).  Each solver keeps its own parameters, sizes, coils and
- * stopping. */
+ * work lists).  Solvers that ran as single solves keep their engines for the
+ * next one, as after pdt_solver_solve.  Each solver keeps its own parameters,
+ * sizes, coils and stopping. */
 PDT_API int pdt_batch_solve(pdt_solver** solvers, int count, int verbose);
 
 /* NEW (no counterpart in the reference, which solves one problem per call,

@@ -179,8 +179,9 @@ __device__ __forceinline__ void store_loss(double ss, double* lpart) {
 // each is read once per strip and not once per tap row.  What bounds it is
 // memory (64 bytes in and 64 out per pixel against 9216 products).  The taps
 // of a pixel are summed in order 0..8.
-// 16 x 320 x 320, 32 -> 32: 50.6 us forward, 57.3 us backward-data (4.1 and
-// 5.5 TB/s on 210 and 315 MB); 163 and 233 us with a wave per 64 pixels, nine
+// 16 x 320 x 320, 32 -> 32: 50 us forward, 57 us backward-data (4.2 and 5.5
+// TB/s on 210 and 315 MB; counted 252 and 371 MB, 5.0 and 6.5 TB/s, with the
+// matrix cores busy 13 us); 163 and 233 us with a wave per 64 pixels, nine
 // fragment loads per 16 pixels and results through LDS.  Rows one step ahead
 // instead of three: 75 and 104 us; shares of 16 rows instead of equal ones (a
 // last round of few waves): 57.6 and 67.4 us.
@@ -653,8 +654,9 @@ __device__ __forceinline__ void grad_partial(const f4 (&acc)[NT], const f4 (&db)
 }
 
 // 32 input channels; COUT 32, or 6 with dz padded to 8 channels.
-// 16 x 320 x 320, 32 -> 32: 60 us, 3.5 TB/s on 210 MB (476 us with single
-// 2-byte LDS reads and 1024 partials).
+// 16 x 320 x 320, 32 -> 32: 60 us for 210 MB of operands, of which the strips'
+// overlapping borders make 283 MB of traffic, 4.7 TB/s; the matrix cores are
+// busy 13 us of it.  (476 us with single 2-byte LDS reads and 1024 partials.)
 template <int COUT>
 __global__ __launch_bounds__(kGradThreads) void wgrad32_kernel(const __bf16* __restrict__ in,
                                                                const __bf16* __restrict__ dz, float* part, int n, int h,

@@ -47,7 +47,9 @@ void cnn_conv_last(hipStream_t st, const void* in, const void* wk, const float* 
 // launch and 0.031 + 0.034 per hidden layer for every thousand pixels.  Depth
 // 5: 1 x 320 x 320 30 against 46 us, 16 x 320 x 320 186 against 255; 1024 x 8
 // x 8 (a third of each strip used, four rounds) 62 against 41; depth 2, 16 x
-// 320 x 320 118 against 72; depth 8, 16 x 320 x 320 516 against 420.
+// 320 x 320 118 against 72; depth 8, 16 x 320 x 320 516 against 420.  Where it
+// takes the slower way: depth 3, 1 x 1000 x 1000 85 against 80; depth 8, 16 x 320
+// x 320 in strips of 81 rows 440 against 409.
 int cnn_net_rows(int depth, int n, int h, int w);
 void cnn_net(hipStream_t st, const CnnLayer* ls, int depth, const float* x, float* y, int n, int h, int w, int rows);
 // The last layer of a training pass: y = conv(in) + b is not stored but

@@ -1460,12 +1460,14 @@ __global__ __launch_bounds__(NT) void k_op_cols_adj(const SliceDev d, SliceDev* 
 // last stage writes T2.  Four barriers and four passes through LDS, where the
 // general kernel has eight and nine.
 // Bound by this chain (descriptor, loads, six stages, stores) with every
-// workgroup resident at once, not by its bytes.  Per launch, general kernel
-// before, this one after: 640 points, 15 coils x 80 columns with the dual step
-// 11.9 -> 10.3 us; 768 points, 15 x 117 16.3 -> 13.4; 512 points in double
-// precision (a runtime plan before), 8 x 64 12.9 -> 8.3.
+// workgroup resident at once, not by its bytes: of a launch of 640 points with
+// the dual step the vector instructions take 2.7 us and the waves wait 49 % of
+// their time.  Per launch, general kernel before, this one after (kernel trace):
+// 640 points, 15 coils x 80 columns with the dual step 12.1 -> 10.6 us; between
+// events, in three passes, 768 points, 15 x 117 15.9 -> 13.1 and 512 points in
+// double precision (a runtime plan before), 8 x 64 11.4 -> 7.5.
 // At most CS columns per group (max_cg): two of 640 points (160 threads) were
-// faster than three or four, 27.8 against 28.4 and 29.0 us per iteration, and
+// faster than three or four, 2 and 4 % of an iteration, and
 // two of 512 in double than four.
 template <class R, int NF>
 struct ColShape {
@@ -1679,9 +1681,11 @@ template <int NT> constexpr int rows_adj_pt() { return NT >= 1024 ? 2 : 4; }
 // The straight-line path loads its sensitivity slots unconditionally, so it
 // is built for as many as it uses: 5 coils for each thread group (15 coils on
 // rows of 320, 20 on rows of 256, 10 on rows of 384 and 512), and for the
-// padded lengths of two groups also 8 (16 coils).  8 slots spill a few
-// registers: 10 coils on rows of 384 take 30.5 us per iteration with them, 28
-// with 5; 12 coils 34 us, against 40 in three passes and k_mri_primal.
+// padded lengths of two groups also 8 (16 coils).  8 slots spill in every paired
+// iteration, 6 registers (28 bytes) on rows of 384 and 21 (88 bytes) on rows of
+// 512, where 5 spill 1 and 13: 10 coils on rows of 384 take 30.5 us per iteration
+// with 8, 28 with 5; 12 coils 34 us, against 40 in three passes and
+// k_mri_primal.
 constexpr int kFusedSlots = 5, kFusedSlotsMore = 8;
 constexpr bool fused_more_ok(int W) { return ct_pad_ok(W) && kRowAdjThreadsWide / W == 2; }
 // Coils per thread group.
@@ -2569,8 +2573,10 @@ static void launch_rows_adj(const Launch& L, bool gap) {
 // and 36.8, 256 x 500, 16 coils (1024 items of four, 1024 places) 51.7 and 49.0,
 // 225 x 500, 20 coils (1125) 63.6 and 72.8; with six or more per CU they need
 // not, 400 x 270, 20 coils 1.08 times faster.  Measured at 982 sizes from 64 x 48
-// to 400 x 700; the rule's choice is at the worst 11 % off the better one, 0.3 %
-// in the mean.
+// to 400 x 700: in single precision and with one_group the rule's choice is at
+// the worst 11 % off the better one, 0.4 % in the mean.  In double precision
+// without one_group four stay the default everywhere, 6 % off in the mean (320 x
+// 400, 6 coils 66.0 and 47.3 with two).
 int default_cb(int dtype, int W, int H, int C, int nc, bool one_group) {
   if (fft_len_compiled(dtype, W)) return kDefaultCb;
   const long twos = long(H) * ((C + 1) / 2), fours = long(H) * ((C + 3) / 4);

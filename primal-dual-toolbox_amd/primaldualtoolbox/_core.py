@@ -291,10 +291,12 @@ def set_tiles(optimizers, cb: int = 0, cg: int = 0, rpi: int = 0, cb_a: int = 0,
 
 
 def batch_profile(optimizers, reps: int = 20) -> list:
-    """profileKernels over the launches of a batch of configured optimizers:
-    per fused kernel, ms per launch over every slice and the algorithmic bytes
-    of that launch summed over the slices.  The iterates are put back after
-    the timing runs."""
+    """profileKernels over the work-list launches of a batch of configured
+    optimizers: per fused kernel, ms per launch over every slice and the
+    algorithmic bytes of that launch summed over the slices.  (A batch that
+    batch_solve runs as concurrent single solves launches what each solver's
+    own profileKernels reports.)  The iterates are put back after the timing
+    runs."""
     for o in optimizers:
         o._push_params()
     arr = (ct.c_void_p * len(optimizers))(*[o._h.value for o in optimizers])
@@ -307,7 +309,8 @@ def batch_profile(optimizers, reps: int = 20) -> list:
 def batch_solve(optimizers, verbose: bool = False) -> None:
     """Solves configured optimizers of one class together: one persistent
     work-list launch per half-iteration for the whole batch, or concurrent
-    single solves where those are faster (large slices, many sizes)."""
+    single solves where those are faster (large slices, many sizes), whose
+    engines the optimizers keep for their next solve."""
     if not optimizers:
         return
     for o in optimizers:
